@@ -4,6 +4,7 @@
 // The per-angle coefficients follow the reference's transferConstants
 // routines; they are computed once per geometry handle (not once per call as
 // in the reference) and kept in device memory.
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdarg>
@@ -233,6 +234,45 @@ void cyl_bp_coeffs(const double *p, CylBPAngle &o) {
 
 }  // namespace
 
+// Column bounds of one direction group.  For a cone the samples of a column
+// at slice s lie at z = s2 + (P2(u, v) - s2) t, t = (s - s0) / (P0(u) - s0): both
+// |V2 t| and the slope |P2 - s2| / |P0 - s0| are largest at corners of the
+// detector and of the slice range, as long as P0 - s0 keeps its sign.
+static ColsBound cols_bound(const Geom3D &g, int dir) {
+    ColsBound b;
+    if (dir > 1 || g.kind == ASTRA_AMD_GEOM_CYLCONE) return b;
+    // a chunk of slices may end up to 3 slices past the volume
+    const double half = 0.5 * (dir == 0 ? g.nx : g.ny) + 3.0;
+    const bool cone = g.kind == ASTRA_AMD_GEOM_CONE;
+    for (unsigned a = 0; a < g.na; ++a) {
+        const FP3DAngle &f = g.fp_host[a];
+        if (f.dir != dir) continue;
+        if (f.v[0] != 0.0 || f.v[1] != 0.0 || f.v[2] == 0.0) return b;
+        if (!cone) {
+            b.spread = std::max(b.spread, std::fabs(f.v[2]));
+            b.typical = std::max(b.typical, std::fabs(f.v[2]));
+            b.slope = std::max(b.slope, std::fabs(f.s[2] / f.s[0]));
+            continue;
+        }
+        const double len = std::sqrt(f.s[0] * f.s[0] + f.s[1] * f.s[1]);
+        double sign = 0.0;
+        for (int c = 0; c < 4; ++c) {
+            const double u = (c & 1) ? g.nu - 1.0 : 0.0, v = (c & 2) ? g.nv - 1.0 : 0.0;
+            const double d = f.p0[0] + u * f.u[0] - f.s[0];
+            if (std::fabs(d) < 1e-3 * (1.0 + len) || d * sign < 0.0) return b;
+            sign = d;
+            const double far = std::max(std::fabs(half - f.s[0]), std::fabs(-half - f.s[0]));
+            b.spread = std::max(b.spread, std::fabs(f.v[2] / d) * far);
+            b.slope = std::max(b.slope,
+                               std::fabs((f.p0[2] + u * f.u[2] + v * f.v[2] - f.s[2]) / d));
+        }
+        const double mid = f.p0[0] + 0.5 * (g.nu - 1.0) * f.u[0] - f.s[0];
+        b.typical = std::max(b.typical, std::fabs(f.v[2] * f.s[0] / mid));
+    }
+    b.ok = std::isfinite(b.spread) && std::isfinite(b.slope);
+    return b;
+}
+
 Geom3D *geom3d_build(int kind, unsigned nx, unsigned ny, unsigned nz, unsigned na, unsigned nu,
                      unsigned nv, const double *vecs, const float *vol_scale) {
     AMX_REQUIRE(kind == ASTRA_AMD_GEOM_CONE || kind == ASTRA_AMD_GEOM_PAR3D ||
@@ -345,6 +385,7 @@ Geom3D *geom3d_build(int kind, unsigned nx, unsigned ny, unsigned nz, unsigned n
     g->zc_default = !cyl && zconst(bd);
     g->zc_fdk = !cyl && zconst(bf);
     g->zc_2d = !cyl && zconst(b2);
+    for (int k = 0; k < 3; ++k) g->cols[k] = cols_bound(*g, k);
     try {
         g->fp = DevArray(sizeof(FP3DAngle) * na);
         g->fp.upload(g->fp_host.data(), sizeof(FP3DAngle) * na);

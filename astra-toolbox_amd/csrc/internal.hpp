@@ -152,6 +152,16 @@ struct Filter {
     DevArray twiddle;  // float2[n_fft]: exp(-2 pi i k / n_fft)
 };
 
+// What the column FP (fp3d_cols.hip) needs to know of a direction group:
+// ok: every angle's detector v axis is the z axis and no ray of the detector
+// runs along a slice; the largest and the typical (volume centre) distance
+// in z, in voxels, of the samples of two neighbouring rays of a column; the
+// largest step in z per slice.
+struct ColsBound {
+    bool ok = false;
+    double spread = 0, typical = 0, slope = 0;
+};
+
 struct Geom3D {
     int kind;  // ASTRA_AMD_GEOM_PAR3D / _CONE / _CYLCONE
     unsigned nx, ny, nz, na, nu, nv;
@@ -168,6 +178,7 @@ struct Geom3D {
     // any angle (nu[2] == dn[2] == 0, e.g. circular cone with a vertical
     // detector), so the BP hoists them out of its z loop
     bool zc_default = false, zc_fdk = false, zc_2d = false;
+    ColsBound cols[3];
     DevArray group_idx[3];               // int[dir_count[k]] angle lists
     // FDK pre-weights [nv][nu] and default Ram-Lak filter, built on first use
     mutable std::mutex fdk_mu;

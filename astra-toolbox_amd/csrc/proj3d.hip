@@ -34,8 +34,7 @@
 #include <cstdlib>
 #include <memory>
 
-#include "devutil.hpp"
-#include "internal.hpp"
+#include "proj3d_dev.hpp"
 
 namespace amx {
 
@@ -191,118 +190,6 @@ __global__ __launch_bounds__(256) void am_to_pairs(const float *__restrict__ src
 }
 
 // ------------------------------------------------------------- FP --------
-struct FPArgs {
-    const float *volp;  // padded slice-major copy of this group
-    unsigned n0, n1, n2;
-    const FP3DAngle *ang;
-    const int *alist;  // angle indices of this direction group
-    unsigned nu, nv, na;
-    float fs1, fs2, osc;
-    float *out;
-    int mode;
-    const float *rb;  // OUT_RESID: b in the output layout
-    const float *rw;  // OUT_RESID: weights in the output layout (may be NULL)
-    int padded_out;   // write [a][v+2][u+2] instead of [v][a][u]
-    // workgroup map (fp_map): detector tiles, angles per block, the range
-    // [lfirst, lfirst + lcount) of alist covered by this launch, and the
-    // part [xfirst[x], xfirst[x + 1]) of that range taken by XCD x
-    unsigned tiles, ablk, lfirst, lcount;
-    unsigned xfirst[9];
-    unsigned ss;  // rays per detector pixel and dimension (DetectorSuperSampling)
-};
-
-// Workgroup -> (detector tile, angle) map.  Workgroups are handed out
-// round-robin over the 8 XCDs (workgroup L runs on XCD L % 8), and each XCD
-// has its own L2.  XCD x takes the angles [xfirst[x], xfirst[x + 1]) of the
-// launch's range (an eighth of them), cut into equal blocks of at most
-// `ablk` angles, in the order (angle block, tile, angle within block); no
-// block spans two XCDs.  The workgroups resident on one XCD at a time are
-// then a few neighbouring tiles, each over a block of consecutive angles,
-// which start together and march through the same slices at the same
-// time: rays of neighbouring angles sample nearly the same voxels, so they
-// share the XCD's L2 instead of each fetching the volume from HBM.
-// Workgroups beyond their XCD's range return at once.  (A single range cut
-// into blocks across the XCDs left the last XCD with the partial block and
-// the others with 48 of every 45 angles' work: 48.7 vs 42.7 ms per group
-// launch at 512^3 / 720 x 768^2.)
-__device__ __forceinline__ bool fp_map_L(const FPArgs &A, unsigned L, unsigned &tile, int &angle) {
-    const unsigned x = L & 7u, q = L >> 3;
-    const unsigned first = A.xfirst[x], count = A.xfirst[x + 1] - first;
-    if (count == 0) return false;
-    const unsigned nblk = (count + A.ablk - 1) / A.ablk;
-    const unsigned bsz = (count + nblk - 1) / nblk;  // angles per block
-    const unsigned span = bsz * A.tiles;             // items per full block
-    const unsigned blk = q / span;
-    const unsigned b0 = blk * bsz;
-    if (b0 >= count) return false;
-    const unsigned bs = min(bsz, count - b0);
-    const unsigned r = q - blk * span;
-    if (r >= bs * A.tiles) return false;
-    tile = r / bs;
-    angle = A.alist[A.lfirst + first + b0 + r % bs];
-    return true;
-}
-
-__device__ __forceinline__ bool fp_map(const FPArgs &A, unsigned &tile, int &angle) {
-    return fp_map_L(A, blockIdx.x, tile, angle);
-}
-
-// One thread per ray; a 256-thread workgroup covers a 16 x 16 detector tile
-// of one angle, each wave a 16 u x 4 v sub-tile.  Ray setup runs in FP64;
-// the slice loop is wave-uniform over the union of the lanes' clipped slice
-// ranges, so the slice base address is scalar and every fetch is one
-// 16-byte load with a 32-bit vector offset.
-// (u, v): detector coordinates of the ray relative to pixel (0, 0)'s centre
-// (fractional for sub-rays).
-// GK: GEO_PAR3D, GEO_CONE (flat detector) or GEO_CYL (cylindrical detector:
-// pixel centre on the cylinder, cuda/3d/cone_cyl.cu:243-258).
-enum { GEO_PAR3D = 0, GEO_CONE = 1, GEO_CYL = 2 };
-
-// The ray of detector coordinates (u, v) in the group's slice frame:
-// texel coordinate - 0.5 along axes 1, 2 at slice s = a_k s + c_k, and the
-// slices [lo, hi] where it can touch the volume.
-template <int GK>
-__device__ __forceinline__ void fp3d_ray_line(const FP3DAngle &G, unsigned nu, unsigned nv,
-                                              unsigned n0, unsigned n1, unsigned n2, double u,
-                                              double v, double &a1, double &a2, double &c1,
-                                              double &c2, int &lo, int &hi) {
-    constexpr bool CONE = GK != GEO_PAR3D;
-    double P[3], d[3];
-    if (GK == GEO_CYL) {
-        const double th = (u - 0.5 * nu + 0.5) * G.dth;
-        const double fv = v - 0.5 * nv + 0.5;
-        const double ct = cos(th), st = sin(th);
-        for (int k = 0; k < 3; ++k) P[k] = G.p0[k] + ct * G.u[k] + st * G.b[k] + fv * G.v[k];
-    } else {
-        for (int k = 0; k < 3; ++k) P[k] = G.p0[k] + u * G.u[k] + v * G.v[k];
-    }
-    for (int k = 0; k < 3; ++k) d[k] = CONE ? (G.s[k] - P[k]) : G.s[k];
-    const double *B = CONE ? G.s : P;
-    a1 = d[1] / d[0];
-    a2 = d[2] / d[0];
-    // texel coordinate - 0.5 at slice s: a_k (s - n0/2 + 0.5 - B0) + B_k + n_k/2 - 0.5
-    const double base = -0.5 * n0 + 0.5 - B[0];
-    c1 = a1 * base + B[1] + 0.5 * n1 - 0.5;
-    c2 = a2 * base + B[2] + 0.5 * n2 - 0.5;
-    lo = 0;
-    hi = (int)n0 - 1;
-    clip_range(a1, c1, (double)n1, (int)n0, lo, hi);
-    clip_range(a2, c2, (double)n2, (int)n0, lo, hi);
-}
-
-template <int GK>
-__device__ __forceinline__ void fp3d_ray(const FPArgs &A, const FP3DAngle &G, double u, double v,
-                                         float &a1f, float &a2f, float &c1f, float &c2f,
-                                         float &scale, int &lo, int &hi) {
-    double a1, a2, c1, c2;
-    fp3d_ray_line<GK>(G, A.nu, A.nv, A.n0, A.n1, A.n2, u, v, a1, a2, c1, c2, lo, hi);
-    a1f = (float)a1;
-    a2f = (float)a2;
-    c1f = (float)(c1 + kPad);  // padded texel coordinates
-    c2f = (float)(c2 + kPad);
-    scale = (float)(sqrt(a1 * a1 * A.fs1 + a2 * a2 * A.fs2 + 1.0) * A.osc);
-}
-
 // Sum of the bilinear samples of slices [slo, shi] (wave-uniform) along the
 // ray (c1, c2) = a s + c through the padded group copy.  Samples at even
 // offsets from slo go to acc0, odd ones to acc1; four loads are issued
@@ -406,25 +293,7 @@ __device__ __forceinline__ void fp3d_item(const FPArgs &A, unsigned L) {
         val /= (float)(R * R);
     }
     if (!active) return;
-    size_t idx = ((size_t)v * A.na + angle) * A.nu + u;
-    size_t oidx = A.padded_out
-                      ? ((size_t)angle * (A.nv + 2 * kPad) + (v + kPad)) * (A.nu + 2 * kPad) + u + kPad
-                      : idx;
-    if (A.mode == OUT_ADD) {
-        A.out[oidx] += val;
-    } else if (A.mode == OUT_SET) {
-        A.out[oidx] = val;
-    } else if (A.mode == OUT_RESID) {  // (b + val) * w
-        float r = A.rb[idx] + val;
-        if (A.rw) r *= A.rw[oidx];
-        A.out[oidx] = r;
-    } else if (A.mode == OUT_RATIO) {
-        A.out[oidx] = em_ratio(A.rb[idx], val);
-    } else {  // OUT_ADDMUL: (out + val) * w
-        float r = A.out[oidx] + val;
-        if (A.rw) r *= A.rw[oidx];
-        A.out[oidx] = r;
-    }
+    fp3d_store(A, u, v, angle, val);
 }
 
 // The FP as a resident grid: workgroup b starts on logical items of XCD
@@ -435,6 +304,10 @@ __device__ __forceinline__ void fp3d_item(const FPArgs &A, unsigned L) {
 // tickets are taken.  The same rays and sums as one workgroup per item
 // (bit for bit), with no XCD left idle while another still has items
 // (41.8 vs 43.0 ms per group launch at 512^3 / 720 x 768^2).
+// The counters are in cache lines of their own, and an exhausted one is read
+// before it is written: 2048 workgroups adding to 8 counters of one line took
+// 0.2 ms however small the projection was.
+constexpr unsigned kTickPitch = 32;  // words from counter to counter
 template <int GK, bool SS>
 __global__ __launch_bounds__(256) void fp3d_kernel(FPArgs A, unsigned *tick, unsigned per_xcd) {
     __shared__ unsigned sh;
@@ -445,10 +318,15 @@ __global__ __launch_bounds__(256) void fp3d_kernel(FPArgs A, unsigned *tick, uns
             unsigned L = 0xffffffffu;
             while (q < 8) {
                 const unsigned x = (home + q) & 7u;
-                const unsigned t = atomicAdd(tick + x, 1u);
-                if (t < per_xcd) {
-                    L = x + 8u * t;
-                    break;
+                unsigned *c = tick + x * kTickPitch;
+                // a counter that has run out is only read: a workgroup that
+                // finds nothing left takes no ticket from any XCD
+                if (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < per_xcd) {
+                    const unsigned t = atomicAdd(c, 1u);
+                    if (t < per_xcd) {
+                        L = x + 8u * t;
+                        break;
+                    }
                 }
                 ++q;
             }
@@ -463,7 +341,7 @@ __global__ __launch_bounds__(256) void fp3d_kernel(FPArgs A, unsigned *tick, uns
 }
 
 __global__ void fp_tick_reset(unsigned *tick) {
-    if (threadIdx.x < 8) tick[threadIdx.x] = 0;
+    if (threadIdx.x < 8) tick[threadIdx.x * kTickPitch] = 0;
 }
 
 // ---- FP with volume slices staged in LDS ---------------------------------
@@ -714,25 +592,7 @@ __global__ __launch_bounds__(256) void fp3d_lds_kernel(FPArgs A) {
         if (angle[j] < 0) continue;
         const float val = (acc0[j] + acc1[j]) * sc[j];
         const int an = angle[j];
-        size_t idx = ((size_t)v * A.na + an) * A.nu + u;
-        size_t oidx = A.padded_out
-                          ? ((size_t)an * (A.nv + 2 * kPad) + (v + kPad)) * (A.nu + 2 * kPad) + u + kPad
-                          : idx;
-        if (A.mode == OUT_ADD) {
-            A.out[oidx] += val;
-        } else if (A.mode == OUT_SET) {
-            A.out[oidx] = val;
-        } else if (A.mode == OUT_RESID) {
-            float r = A.rb[idx] + val;
-            if (A.rw) r *= A.rw[oidx];
-            A.out[oidx] = r;
-        } else if (A.mode == OUT_RATIO) {
-            A.out[oidx] = em_ratio(A.rb[idx], val);
-        } else {
-            float r = A.out[oidx] + val;
-            if (A.rw) r *= A.rw[oidx];
-            A.out[oidx] = r;
-        }
+        fp3d_store(A, u, v, an, val);
     }
 }
 
@@ -1603,49 +1463,6 @@ unsigned bp_achunk(size_t pair_bytes, unsigned na) {
     return (unsigned)((na + chunks - 1) / chunks);
 }
 
-// Most angles per block of the FP workgroup map (fp_map): an XCD's range
-// is cut into equal blocks of at most this many angles.
-// ASTRA_AMD_FP3D_ANGLE_BLOCK overrides the default 64 (1..64; read at every
-// call).  Measured at 512^3 / 720 x 768^2 (45 angles per XCD and group),
-// ms per group launch: 16: 43.5, 23: 42.9, 32 (blocks of 32 and 13): 44.0,
-// 45 or 64 (one block): 42.8, 42.7.
-unsigned fp_angle_block() {
-    const char *e = std::getenv("ASTRA_AMD_FP3D_ANGLE_BLOCK");
-    const long x = e ? std::strtol(e, nullptr, 10) : 0;
-    return (x >= 1 && x <= 64) ? (unsigned)x : 64u;
-}
-
-// Split the angles [first, first + count) of a group's list over the 8
-// XCDs in equal counts: xfirst[x] is the first angle of XCD x (relative to
-// `first`), xfirst[8] = count.  (Splitting by an estimated cost per angle
-// -- samples, or cache lines fetched -- measured slower at 512^3 / 720 x
-// 768^2: 44.5-45.9 against 43.8-44.3 ms per group launch; the per-angle time
-// varies less with the angle than either estimate.)
-void xcd_split(unsigned count, unsigned (&xfirst)[9]) {
-    for (unsigned x = 0; x <= 8; ++x) xfirst[x] = (unsigned)((size_t)count * x / 8);
-}
-
-// Launch `kern` over the angles of one direction group, in as many
-// launches as the 2^32 work-item limit of one grid requires.
-template <typename K>
-void fp_group_launches(FPArgs A, unsigned count, K kern, hipStream_t s) {
-    A.tiles = ((A.nu + 15) / 16) * ((A.nv + 15) / 16);
-    A.ablk = fp_angle_block();
-    const size_t max_groups = (1u << 24) - 8;  // 256 threads each
-    AMX_REQUIRE((size_t)A.tiles * 16 <= max_groups, "fp3d: detector too large for one launch");
-    // at most max_groups / tiles - 8 angles per launch: 8 XCD ranges of
-    // ceil(count / 8) angles fit
-    const unsigned per_launch = (unsigned)(max_groups / A.tiles - 8);
-    for (unsigned first = 0; first < count; first += per_launch) {
-        A.lfirst = first;
-        A.lcount = std::min(count - first, per_launch);
-        xcd_split(A.lcount, A.xfirst);
-        const size_t groups = (size_t)8 * ((A.lcount + 7) / 8) * A.tiles;
-        kern(A, (unsigned)groups);
-        AMX_LAUNCHED();
-    }
-}
-
 // One resident-grid FP launch over `groups` logical workgroups (8 x the
 // items per XCD): clear the ticket counters (a kernel, so the launch can be
 // captured), then as many workgroups as are resident at once (a multiple
@@ -1672,7 +1489,7 @@ void fp_resident_launch(void (*kern)(FPArgs, unsigned *, unsigned), const FPArgs
     }
     fp_tick_reset<<<1, 64, 0, s>>>(tick);
     AMX_LAUNCHED();
-    kern<<<grid, 256, 0, s>>>(a, tick, groups / 8);
+    kern<<<std::min(grid, groups), 256, 0, s>>>(a, tick, groups / 8);
 }
 
 // ASTRA_AMD_FP3D_LDS=1: the FP stages volume slices in LDS for groups of
@@ -1723,24 +1540,39 @@ void fp3d_launch(const Geom3D &g, const float *vol, float *proj, float out_scale
     // the cylindrical-detector FP has no sub-rays (ConeCylFP ignores
     // iRaysPerDetDim, cuda/3d/cone_cyl.cu:613-666)
     if (g.kind == ASTRA_AMD_GEOM_CYLCONE) ss = 1;
+    // groups whose detector columns run along z take the column FP
+    // (ASTRA_AMD_FP3D_LDS, when set, picks one of the gather's two forms)
+    const bool cols_on = ss == 1 && !std::getenv("ASTRA_AMD_FP3D_LDS");
     size_t need = 0;
-    int groups[3], ng = 0;
+    int groups[3], ng = 0, rays[3] = {0, 0, 0};
+    bool cols = false;
     for (int k = 0; k < 3; ++k)
         if (g.dir_count[k]) {
-            need = std::max(need, group_elems(g, k));
+            rays[k] = cols_on ? fp3d_cols_rays(g, k) : 0;
+            if (rays[k])
+                cols = true;
+            else
+                need = std::max(need, group_elems(g, k) * sizeof(float2));
             groups[ng++] = k;
         }
-    Scratch copy(need * sizeof(float2), s);  // row-pair copy
-    Scratch tick(8 * sizeof(unsigned), s);    // ticket counters of the resident FP grid
+    std::unique_ptr<Scratch> colv, copy, tick;
+    if (cols) {
+        colv.reset(new Scratch(fp3d_cols_bytes(g), s));
+        fp3d_cols_copy(g, vol, colv->as<float>(), s);
+    }
+    if (need) {
+        copy.reset(new Scratch(need, s));                  // row-pair copy
+        tick.reset(new Scratch(8 * kTickPitch * sizeof(unsigned), s));  // ticket counters of the resident FP grid
+    }
     for (int i = 0; i < ng; ++i) {
         const int k = groups[i];
-        make_group_copy(g, k, vol, copy.as<float2>(), s);
+        if (!rays[k]) make_group_copy(g, k, vol, copy->as<float2>(), s);
         FPArgs A = fp_args(g, k, out_scale);
         // march3d's buffer loads address a slice at 32-bit scalar offsets
         // of up to 3 slices
         AMX_REQUIRE((size_t)(A.n1 + 2 * kPad) * (A.n2 + 2 * kPad) * sizeof(float2) <= (1ull << 30),
                     "fp3d: volume slice too large (%u x %u)", A.n1, A.n2);
-        A.volp = copy.as<float>();
+        A.volp = rays[k] ? nullptr : copy->as<float>();
         A.out = proj;
         A.rb = resid_b;
         A.rw = resid_w;
@@ -1753,27 +1585,32 @@ void fp3d_launch(const Geom3D &g, const float *vol, float *proj, float out_scale
                                                                      : "fp3d_par3d",
                                   (double)g.dir_count[k] * g.nu * g.nv * A.n0 * ss * ss, s);
         A.ss = ss;
+        if (rays[k]) {
+            fp3d_cols_launch(g, k, rays[k], A, colv->as<float>(), s);
+            prof_end(pt, s);
+            continue;
+        }
         if (ss == 1 && g.kind != ASTRA_AMD_GEOM_CYLCONE && fp_lds()) {
             fp_lds_launches(A, g.dir_count[k], g.kind == ASTRA_AMD_GEOM_CONE, s);
             prof_end(pt, s);
             continue;
         }
-        fp_group_launches(A, g.dir_count[k], [&](const FPArgs &a, unsigned groups) {
+        fp_group_launches(A, fp_tiles(A), (unsigned)g.dir_count[k], [&](const FPArgs &a, unsigned groups) {
             // groups = 8 x the items per XCD
             if (g.kind == ASTRA_AMD_GEOM_CYLCONE)
-                fp_resident_launch(fp3d_kernel<GEO_CYL, false>, a, tick.as<unsigned>(), groups, s);
+                fp_resident_launch(fp3d_kernel<GEO_CYL, false>, a, tick->as<unsigned>(), groups, s);
             else if (ss > 1) {
                 if (g.kind == ASTRA_AMD_GEOM_CONE)
-                    fp_resident_launch(fp3d_kernel<GEO_CONE, true>, a, tick.as<unsigned>(), groups, s);
+                    fp_resident_launch(fp3d_kernel<GEO_CONE, true>, a, tick->as<unsigned>(), groups, s);
                 else
-                    fp_resident_launch(fp3d_kernel<GEO_PAR3D, true>, a, tick.as<unsigned>(), groups,
+                    fp_resident_launch(fp3d_kernel<GEO_PAR3D, true>, a, tick->as<unsigned>(), groups,
                                        s);
             } else {
                 if (g.kind == ASTRA_AMD_GEOM_CONE)
-                    fp_resident_launch(fp3d_kernel<GEO_CONE, false>, a, tick.as<unsigned>(), groups,
+                    fp_resident_launch(fp3d_kernel<GEO_CONE, false>, a, tick->as<unsigned>(), groups,
                                        s);
                 else
-                    fp_resident_launch(fp3d_kernel<GEO_PAR3D, false>, a, tick.as<unsigned>(), groups,
+                    fp_resident_launch(fp3d_kernel<GEO_PAR3D, false>, a, tick->as<unsigned>(), groups,
                                        s);
             }
         }, s);
@@ -1791,7 +1628,7 @@ void fp3d_sumsq_launch(const Geom3D &g, float *proj, float out_scale, int mode, 
         A.out = proj;
         A.mode = mode;
         A.ss = 1;
-        fp_group_launches(A, g.dir_count[k], [&](const FPArgs &a, unsigned groups) {
+        fp_group_launches(A, fp_tiles(A), (unsigned)g.dir_count[k], [&](const FPArgs &a, unsigned groups) {
             fp3d_sumsq_kernel<<<groups, 256, 0, s>>>(a);
         }, s);
     }
