@@ -244,6 +244,7 @@ static ColsBound cols_bound(const Geom3D &g, int dir) {
     // a chunk of slices may end up to 3 slices past the volume
     const double half = 0.5 * (dir == 0 ? g.nx : g.ny) + 3.0;
     const bool cone = g.kind == ASTRA_AMD_GEOM_CONE;
+    b.closest = INFINITY;
     for (unsigned a = 0; a < g.na; ++a) {
         const FP3DAngle &f = g.fp_host[a];
         if (f.dir != dir) continue;
@@ -251,6 +252,7 @@ static ColsBound cols_bound(const Geom3D &g, int dir) {
         if (!cone) {
             b.spread = std::max(b.spread, std::fabs(f.v[2]));
             b.typical = std::max(b.typical, std::fabs(f.v[2]));
+            b.closest = std::min(b.closest, std::fabs(f.v[2]));
             b.slope = std::max(b.slope, std::fabs(f.s[2] / f.s[0]));
             continue;
         }
@@ -262,7 +264,9 @@ static ColsBound cols_bound(const Geom3D &g, int dir) {
             if (std::fabs(d) < 1e-3 * (1.0 + len) || d * sign < 0.0) return b;
             sign = d;
             const double far = std::max(std::fabs(half - f.s[0]), std::fabs(-half - f.s[0]));
+            const double near = std::fabs(f.s[0]) > half ? std::fabs(f.s[0]) - half : 0.0;
             b.spread = std::max(b.spread, std::fabs(f.v[2] / d) * far);
+            b.closest = std::min(b.closest, std::fabs(f.v[2] / d) * near);
             b.slope = std::max(b.slope,
                                std::fabs((f.p0[2] + u * f.u[2] + v * f.v[2] - f.s[2]) / d));
         }

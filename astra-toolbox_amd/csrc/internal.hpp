@@ -155,11 +155,12 @@ struct Filter {
 // What the column FP (fp3d_cols.hip) needs to know of a direction group:
 // ok: every angle's detector v axis is the z axis and no ray of the detector
 // runs along a slice; the largest and the typical (volume centre) distance
-// in z, in voxels, of the samples of two neighbouring rays of a column; the
-// largest step in z per slice.
+// in z, in voxels, of the samples of two neighbouring rays of a column, and
+// the smallest (0: they meet inside the volume); the largest step in z per
+// slice.
 struct ColsBound {
     bool ok = false;
-    double spread = 0, typical = 0, slope = 0;
+    double spread = 0, typical = 0, closest = 0, slope = 0;
 };
 
 struct Geom3D {

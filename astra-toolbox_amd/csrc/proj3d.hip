@@ -1824,16 +1824,62 @@ void bp3d_matched_launch(const Geom3D &g, const float *proj, float *vol, float o
     // (one angle at least): the tables are scratch of every gradient step
     // of the differentiable projector, so they stay small beside the data
     const size_t per_angle = NU * NV * (sizeof(float4) + sizeof(float));
-    const unsigned chunk = (unsigned)std::max<size_t>(
-        1, std::min<size_t>(g.na, (size_t(128) << 20) / per_angle));
+    const size_t per_angle_cols = NU * (NV * sizeof(float) + sizeof(float4) + sizeof(float2));
+    auto chunk_of = [&](size_t per) {
+        const size_t n = std::min<size_t>(g.na, (size_t(128) << 20) / per);
+        return (unsigned)std::max<size_t>(1, std::min<size_t>(n, 32768));
+    };
     const bool cyl = g.kind == ASTRA_AMD_GEOM_CYLCONE;
-    Scratch rays(per_angle * chunk, s), geo((size_t)chunk * 3 * sizeof(float4), s);
-    float4 *rp = rays.as<float4>();
-    float *yp = reinterpret_cast<float *>(rp + NU * NV * chunk);
+    // groups whose detector columns run along z split into a pass over u and
+    // one over v (ASTRA_AMD_MATCHED_SLICES, when set, asks for the general
+    // gather); their sums are kept z-fastest and added to vol at the end
+    const bool cols_on = ss == 1 && !cyl && !std::getenv("ASTRA_AMD_MATCHED_SLICES");
+    bool cols[3], any_cols = false, any_gather = false;
+    for (int k = 0; k < 3; ++k) {
+        cols[k] = cols_on && g.dir_count[k] && adj3d_cols_ok(g, k);
+        any_cols |= cols[k];
+        any_gather |= g.dir_count[k] && !cols[k];
+    }
+    size_t bytes = 0;
+    unsigned most = 1;
+    if (any_gather) {
+        bytes = per_angle * chunk_of(per_angle);
+        most = chunk_of(per_angle);
+    }
+    if (any_cols) {
+        bytes = std::max(bytes, per_angle_cols * chunk_of(per_angle_cols));
+        most = std::max(most, chunk_of(per_angle_cols));
+    }
+    Scratch rays(bytes, s), geo((size_t)most * 3 * sizeof(float4), s);
+    std::unique_ptr<Scratch> colv;
+    if (any_cols) {
+        colv.reset(new Scratch(nvox * sizeof(float), s));
+        fill_launch(colv->as<float>(), nvox, 0.f, s);
+    }
     for (int k = 0; k < 3; ++k) {
         if (!g.dir_count[k]) continue;
+        const unsigned chunk = chunk_of(cols[k] ? per_angle_cols : per_angle);
         FPArgs A = fp_args(g, k, out_scale);
         A.ss = ss;
+        if (cols[k]) {
+            float4 *q0 = rays.as<float4>();
+            float2 *q1 = reinterpret_cast<float2 *>(q0 + NU * chunk);
+            float *yw = reinterpret_cast<float *>(q1 + NU * chunk);
+            for (unsigned first = 0; first < (unsigned)g.dir_count[k]; first += chunk) {
+                A.lfirst = first;
+                A.lcount = std::min((unsigned)g.dir_count[k] - first, chunk);
+                const unsigned gb = (A.lcount + 63) / 64;
+                if (g.kind == ASTRA_AMD_GEOM_CONE)
+                    matched_geo_kernel<true><<<gb, 64, 0, s>>>(A, geo.as<float4>());
+                else
+                    matched_geo_kernel<false><<<gb, 64, 0, s>>>(A, geo.as<float4>());
+                AMX_LAUNCHED();
+                adj3d_cols_launch(g, k, A, proj, geo.as<float4>(), q0, q1, yw, colv->as<float>(), s);
+            }
+            continue;
+        }
+        float4 *rp = rays.as<float4>();
+        float *yp = reinterpret_cast<float *>(rp + NU * NV * chunk);
         MatchedArgs M{};
         M.rays = rp;
         M.yw = yp;
@@ -1883,6 +1929,7 @@ void bp3d_matched_launch(const Geom3D &g, const float *proj, float *vol, float o
             AMX_LAUNCHED();
         }
     }
+    if (any_cols) adj3d_cols_add(g, colv->as<float>(), vol, s);
 }
 
 }  // namespace amx
