@@ -641,63 +641,6 @@ __global__ __launch_bounds__(256) void fp3d_sumsq_kernel(FPArgs A) {
 }
 
 // ------------------------------------------------------------- BP --------
-struct BPArgs {
-    const float *pp;  // padded angle-major projections
-    unsigned nu, nv, na;
-    const BP3DAngle *ang;
-    const float *aw;  // par3d per-angle weights
-    unsigned nx, ny, nz;
-    float osc;
-    float *vol;
-    int mode;
-    const float *uw;  // OUT_UPDATE: per-voxel weights (may be NULL)
-    float lo, hi;     // OUT_UPDATE: clamp
-    const float *pre; // bp3d_kernel: BP of earlier angle chunks, added before the epilogue (or NULL)
-};
-
-// Epilogue of a column of ZS voxels: scale, add the earlier chunks, write
-// in the launch's mode.
-// Every load of the column (earlier chunks, old values, weights) is issued
-// before the first store, so the column's read-modify-write costs one
-// memory round trip, not one per voxel (the compiler cannot reorder a load
-// of vol after a store to vol by itself).  Z0 is the workgroup's, so the
-// bounds tests are uniform.
-template <int ZS>
-__device__ __forceinline__ void bp_column_store(const BPArgs &A, int X, int Y, int Z0,
-                                                const float (&acc)[ZS]) {
-    const int nzr = min(ZS, (int)A.nz - Z0);
-    const size_t plane = (size_t)A.ny * A.nx;
-    const size_t base = ((size_t)Z0 * A.ny + Y) * A.nx + X;
-    const bool old = A.mode != OUT_SET;
-    const bool wts = (A.mode == OUT_EMUPD || A.mode == OUT_UPDATE) && A.uw;
-    float pv[ZS], ov[ZS], wv[ZS];
-#pragma unroll
-    for (int i = 0; i < ZS; ++i) {
-        pv[i] = 0.f;
-        ov[i] = 0.f;
-        wv[i] = 1.f;
-        if (i < nzr) {
-            const size_t idx = base + i * plane;
-            if (A.pre) pv[i] = A.pre[idx];
-            if (old) ov[i] = A.vol[idx];
-            if (wts) wv[i] = A.uw[idx];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < ZS; ++i) {
-        if (i < nzr) {
-            float val = acc[i] * A.osc;
-            if (A.pre) val += pv[i];
-            float out;
-            if (A.mode == OUT_ADD) out = ov[i] + val;
-            else if (A.mode == OUT_SET) out = val;
-            else if (A.mode == OUT_EMUPD) out = ov[i] * (val * wv[i]);
-            else out = fminf(fmaxf(fmaf(wv[i], val, ov[i]), A.lo), A.hi);  // OUT_UPDATE
-            A.vol[base + i * plane] = out;
-        }
-    }
-}
-
 // KIND: 0 cone fr^2 (default / FDK), 1 cone fr (2D weighting), 2 par3d.
 // One thread per (x, y) column of ZS voxels; 16 x 16 threads per group.
 // The angle loop is uniform, so the per-angle coefficients are scalar loads
@@ -707,13 +650,10 @@ __device__ __forceinline__ void bp_column_store(const BPArgs &A, int X, int Y, i
 // tap offset and weight and the voxel weight are then computed once per
 // column and angle.  Both forms take the same fp32 operations on the same
 // values (adding a zero increment is exact), so they give identical results.
+// Sums over the angles a0, a0 + step, ... of the launch.
 template <int KIND, int ZS, bool ZC>
-__global__ __launch_bounds__(256) void bp3d_kernel(BPArgs A) {
-    const unsigned tiles_x = (A.nx + 15) / 16;
-    const int X = (blockIdx.x % tiles_x) * 16 + (threadIdx.x & 15);
-    const int Y = (blockIdx.x / tiles_x) * 16 + (threadIdx.x >> 4);
-    const int Z0 = blockIdx.y * ZS;
-    if (X >= (int)A.nx || Y >= (int)A.ny) return;
+__device__ __forceinline__ void bp_gather_column(const BPArgs &A, int X, int Y, int Z0, unsigned a0, unsigned step,
+                                                 float (&acc)[ZS]) {
     const float fx = X - 0.5f * A.nx + 0.5f;
     const float fy = Y - 0.5f * A.ny + 0.5f;
     const float fz = Z0 - 0.5f * A.nz + 0.5f;
@@ -721,12 +661,11 @@ __global__ __launch_bounds__(256) void bp3d_kernel(BPArgs A) {
     const size_t plane = (size_t)(A.nv + 2 * kPad) * pitch * 2; // floats per angle
     const unsigned rowb = pitch * 8u;                           // bytes per row
     const float hiu = (float)A.nu + 2.5f, hiv = (float)A.nv + 2.5f;
-    float acc[ZS];
 #pragma unroll
     for (int i = 0; i < ZS; ++i) acc[i] = 0.f;
 
-    const float *pl = A.pp;
-    for (unsigned a = 0; a < A.na; ++a, pl += plane) {
+    const float *pl = A.pp + a0 * plane;
+    for (unsigned a = a0; a < A.na; a += step, pl += step * plane) {
         const BP3DAngle c = A.ang[a];
         float un = fmaf(fz, c.nu[2], fmaf(fy, c.nu[1], fmaf(fx, c.nu[0], c.nu[3])));
         float vn = fmaf(fz, c.nv[2], fmaf(fy, c.nv[1], fmaf(fx, c.nv[0], c.nv[3])));
@@ -769,189 +708,53 @@ __global__ __launch_bounds__(256) void bp3d_kernel(BPArgs A) {
             }
         }
     }
+}
+
+template <int KIND, int ZS, bool ZC>
+__global__ __launch_bounds__(256) void bp3d_kernel(BPArgs A) {
+    const unsigned tiles_x = (A.nx + 15) / 16;
+    const int X = (blockIdx.x % tiles_x) * 16 + (threadIdx.x & 15);
+    const int Y = (blockIdx.x / tiles_x) * 16 + (threadIdx.x >> 4);
+    const int Z0 = blockIdx.y * ZS;
+    if (X >= (int)A.nx || Y >= (int)A.ny) return;
+    float acc[ZS];
+    bp_gather_column<KIND, ZS, ZC>(A, X, Y, Z0, 0, 1, acc);
     bp_column_store<ZS>(A, X, Y, Z0, acc);
 }
 
-// ---- BP with the detector footprint staged in LDS -----------------------
-// The z-constant BP above reads one 16-byte tap (two difference pairs) per
-// voxel and angle through the texture-address path, which bounds it.  Here
-// each workgroup (16 x 16 columns of ZS voxels) stages, per angle, the
-// rectangle of the pair plane that its block projects into as 16-byte
-// quads -- quad (r, c) = pairs (r, c) and (r, c + 1), the whole tap -- so
-// that every tap is one aligned 16-byte LDS read.  Thread t stages column
-// t % 64 of rows t / 64 + 4 k (k < 8) with 16-byte loads issued one angle
-// ahead and held in registers while the current angle is sampled, so the
-// staging needs no index division.  The footprint is the bounding box of
-// the projected corners of the block (u and v are linear-fractional in the
-// voxel position, so the extremes over the block are at its corners; the
-// clamp to the padded range is monotone), widened by one texel on each
-// side, far beyond the fp32 rounding of the taps (replayed on the CPU over
-// whole geometries by the tests).  Taps, weights and the order of the sums
-// are those of bp3d_kernel<KIND, ZS, true>, so both give the same floats.
-// An angle whose footprint exceeds 64 quads x 32 rows or the tile, or whose
-// denominator changes sign over the block, is sampled from global memory
-// as in bp3d_kernel.  A staged row is `lp` quads long: lp = w | 1 (pm < 0)
-// or w + ((pm - w) mod 16) (pm in [0, 16)), so that rows start at
-// different offsets modulo the 16 quads (256 bytes) of one LDS cycle.
-constexpr int kTileCap = 2048;   // LDS quads of the staged tile (32 KiB)
-constexpr int kFpGroup = 256;    // angles whose footprints are held at once
-constexpr int kStageCols = 64;   // widest staged footprint (quads)
-constexpr int kStageRows = 32;   // tallest staged footprint (rows): 4 per thread slot
-constexpr int kStageSlots = kStageRows / 4;
-
-__device__ __forceinline__ int lds_row_pitch(int w, int pm) {
-    return pm < 0 ? (w | 1) : w + ((pm - w) & 15);
-}
-
-template <int KIND>
-__device__ int4 bp_footprint(const BP3DAngle &c, float x0, float x1, float y0, float y1, float z0,
-                             float z1, float hiu, float hiv, int pitch, int prow, int pm) {
-    float umin = INFINITY, umax = -INFINITY, vmin = INFINITY, vmax = -INFINITY;
-    float dmin = INFINITY, dmax = -INFINITY;
-    for (int j = 0; j < 4; ++j) {
-        const float x = (j & 1) ? x1 : x0, y = (j & 2) ? y1 : y0;
-        const float un = fmaf(y, c.nu[1], fmaf(x, c.nu[0], c.nu[3]));
-        const float dn = fmaf(y, c.dn[1], fmaf(x, c.dn[0], c.dn[3]));
-        dmin = fminf(dmin, dn);
-        dmax = fmaxf(dmax, dn);
-        const float fr = (KIND == 2) ? 1.f : 1.f / dn;
-        const float pu = clamp_pad(un * fr, hiu);
-        umin = fminf(umin, pu);
-        umax = fmaxf(umax, pu);
-        for (int k = 0; k < 2; ++k) {
-            const float z = k ? z1 : z0;
-            const float vn = fmaf(z, c.nv[2], fmaf(y, c.nv[1], fmaf(x, c.nv[0], c.nv[3])));
-            const float pv = clamp_pad(vn * fr, hiv);
-            vmin = fminf(vmin, pv);
-            vmax = fmaxf(vmax, pv);
-        }
-    }
-    const bool sign_ok = (KIND == 2) || dmin > 0.f || dmax < 0.f;
-    const bool finite = __builtin_isfinite(umin) && __builtin_isfinite(umax) &&
-                        __builtin_isfinite(vmin) && __builtin_isfinite(vmax);
-    if (!sign_ok || !finite) return make_int4(0, 0, 0, 0);
-    // taps: quad floor(pu) (pairs floor(pu), floor(pu) + 1) of pair row
-    // floor(pv); one texel of margin on each side.  Quad c reads pairs c and
-    // c + 1, so the last quad column is at most pitch - 2.
-    const int u0 = max(0, (int)umin - 1), u1 = min(pitch - 2, (int)umax + 1);
-    const int v0 = max(0, (int)vmin - 1), v1 = min(prow - 1, (int)vmax + 1);
-    const int w = u1 - u0 + 1, h = v1 - v0 + 1;
-    if (w < 1 || w > kStageCols || h > kStageRows || lds_row_pitch(w, pm) * h > kTileCap)
-        return make_int4(0, 0, 0, 0);
-    return make_int4(u0, v0, w, h);
-}
-
-template <int KIND, int ZS>
-__global__ __launch_bounds__(256) void bp3d_lds_kernel(BPArgs A, int pm) {
-    __shared__ float4 tile[kTileCap];
-    __shared__ int4 fps[kFpGroup];
-    const unsigned tid = threadIdx.x;
-    const unsigned tiles_x = (A.nx + 15) / 16;
-    const int X0 = (blockIdx.x % tiles_x) * 16, Y0 = (blockIdx.x / tiles_x) * 16;
-    const int X = X0 + (int)(tid & 15);
-    const int Y = Y0 + (int)(tid >> 4);
+// The same for volumes too small to fill the chip: each of a workgroup's 4
+// waves takes every fourth angle of the same 8 x 8 columns, and the first
+// wave adds their sums in the order of the waves.  A call's time here is one
+// wave's chain of angles (a load's latency each), so a quarter of the
+// angles, and four times the waves.  64^3 / 90 x 96^2: 96 us as 64 workgroups
+// of bp3d_kernel, 22 as 1024 of these.
+constexpr int kSplitZ = 4;
+template <int KIND, bool ZC>
+__global__ __launch_bounds__(256) void bp3d_split_kernel(BPArgs A) {
+    constexpr int ZS = kSplitZ;
+    __shared__ float part[3][ZS][64];
+    const unsigned tiles_x = (A.nx + 7) / 8;
+    const int lane = threadIdx.x & 63;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int X = (blockIdx.x % tiles_x) * 8 + (lane & 7);
+    const int Y = (blockIdx.x / tiles_x) * 8 + (lane >> 3);
     const int Z0 = blockIdx.y * ZS;
-    const bool active = X < (int)A.nx && Y < (int)A.ny;
-    const float hx = 0.5f * A.nx - 0.5f, hy = 0.5f * A.ny - 0.5f, hz = 0.5f * A.nz - 0.5f;
-    const float fx = X - 0.5f * A.nx + 0.5f;
-    const float fy = Y - 0.5f * A.ny + 0.5f;
-    const float fz = Z0 - 0.5f * A.nz + 0.5f;
-    // corners of the block's voxel centres (the columns inside the volume,
-    // all ZS slices: the slices past nz are computed and discarded)
-    const float cx0 = X0 - hx, cx1 = min(X0 + 15, (int)A.nx - 1) - hx;
-    const float cy0 = Y0 - hy, cy1 = min(Y0 + 15, (int)A.ny - 1) - hy;
-    const float cz0 = Z0 - hz, cz1 = (Z0 + ZS - 1) - hz;
-    const unsigned pitch = A.nu + 2 * kPad;                    // pairs per row
-    const unsigned prow = A.nv + 2 * kPad;                     // rows per angle
-    const size_t plane = (size_t)prow * pitch;                 // pairs per angle
-    const unsigned rowb = pitch * 8u;
-    const float hiu = (float)A.nu + 2.5f, hiv = (float)A.nv + 2.5f;
-    const int sc = (int)(tid & 63), sr = (int)(tid >> 6);       // staging column, first row
-    const char *tile_b = reinterpret_cast<const char *>(tile);
+    const bool in = X < (int)A.nx && Y < (int)A.ny;
     float acc[ZS];
 #pragma unroll
     for (int i = 0; i < ZS; ++i) acc[i] = 0.f;
-    float4 pre[kStageSlots];
-
-    // this thread's quads of the footprint: column sc of rows sr + 4 k
-    auto fetch = [&](unsigned a, int4 f) {
-        const float *pl = A.pp + (size_t)a * plane * 2;
-        unsigned off = ((unsigned)(f.y + sr) * pitch + (unsigned)(f.x + sc)) * 8u;
-        const unsigned step = 4u * rowb;
+    if (in) bp_gather_column<KIND, ZS, ZC>(A, X, Y, Z0, wave, 4, acc);
+    if (wave) {
 #pragma unroll
-        for (int k = 0; k < kStageSlots; ++k, off += step)
-            if (sc < f.z && sr + 4 * k < f.w) pre[k] = ld4b(pl, off);
-    };
-
-    for (unsigned g0 = 0; g0 < A.na; g0 += kFpGroup) {
-        const unsigned gn = min((unsigned)kFpGroup, A.na - g0);
-        __syncthreads();  // the previous group's footprints and tile are no longer read
-        if (tid < gn)
-            fps[tid] = bp_footprint<KIND>(A.ang[g0 + tid], cx0, cx1, cy0, cy1, cz0, cz1, hiu, hiv,
-                                          (int)pitch, (int)prow, pm);
-        __syncthreads();
-        if (fps[0].z) fetch(g0, fps[0]);
-        for (unsigned k = 0; k < gn; ++k) {
-            const unsigned a = g0 + k;
-            const int4 f = fps[k];
-            const int lp = lds_row_pitch(f.z, pm);
-            if (k) __syncthreads();  // every thread is done with angle a - 1's tile
-            if (f.z) {
-                int idx = sr * lp + sc;
-#pragma unroll
-                for (int j = 0; j < kStageSlots; ++j, idx += 4 * lp)
-                    if (sc < f.z && sr + 4 * j < f.w) tile[idx] = pre[j];
-            }
-            __syncthreads();  // the tile holds angle a
-            if (k + 1 < gn) {
-                const int4 fn = fps[k + 1];
-                if (fn.z) fetch(a + 1, fn);
-            }
-            if (!active) continue;
-            const BP3DAngle c = A.ang[a];
-            const float un = fmaf(fz, c.nu[2], fmaf(fy, c.nu[1], fmaf(fx, c.nu[0], c.nu[3])));
-            float vn = fmaf(fz, c.nv[2], fmaf(fy, c.nv[1], fmaf(fx, c.nv[0], c.nv[3])));
-            const float dn = fmaf(fz, c.dn[2], fmaf(fy, c.dn[1], fmaf(fx, c.dn[0], c.dn[3])));
-            const float wa = (KIND == 2) ? A.aw[a] : 1.f;
-            const float fr = (KIND == 2) ? 1.f : __builtin_amdgcn_rcpf(dn);
-            const float pu = clamp_pad(un * fr, hiu);
-            const float wu = frac(pu);
-            const float wgt = (KIND == 0) ? fr * fr : (KIND == 1 ? fr : wa);
-            if (f.z) {
-                // byte offset of tap row r: r * lp * 16 + (column - u0 - v0 lp) * 16;
-                // inside the tile by the footprint's margin
-                const int lp16 = lp * 16;
-                const int base = ((int)(unsigned)pu - f.x - f.y * lp) * 16;
-                float4 q[ZS];
-                float wv[ZS];
-#pragma unroll
-                for (int i = 0; i < ZS; ++i) {
-                    const float pv = clamp_pad(vn * fr, hiv);
-                    wv[i] = frac(pv);
-                    const int off = __mul24((int)(unsigned)pv, lp16) + base;
-                    q[i] = *reinterpret_cast<const float4 *>(tile_b + off);
-                    vn += c.nv[2];
-                }
-#pragma unroll
-                for (int i = 0; i < ZS; ++i) acc[i] = fmaf(wgt, bilerp_pairs(q[i], wu, wv[i]), acc[i]);
-            } else {
-                const float *pl = A.pp + (size_t)a * plane * 2;
-                const unsigned ou = (unsigned)pu << 3;
-                float4 q[ZS];
-                float wv[ZS];
-#pragma unroll
-                for (int i = 0; i < ZS; ++i) {
-                    const float pv = clamp_pad(vn * fr, hiv);
-                    wv[i] = frac(pv);
-                    q[i] = ld4b(pl, __umul24((unsigned)pv, rowb) + ou);
-                    vn += c.nv[2];
-                }
-#pragma unroll
-                for (int i = 0; i < ZS; ++i) acc[i] = fmaf(wgt, bilerp_pairs(q[i], wu, wv[i]), acc[i]);
-            }
-        }
+        for (int i = 0; i < ZS; ++i) part[wave - 1][i][lane] = acc[i];
     }
-    if (active) bp_column_store<ZS>(A, X, Y, Z0, acc);
+    __syncthreads();
+    if (wave || !in) return;
+#pragma unroll
+    for (int w = 0; w < 3; ++w)
+#pragma unroll
+        for (int i = 0; i < ZS; ++i) acc[i] += part[w][i][lane];
+    bp_column_store<ZS>(A, X, Y, Z0, acc);
 }
 
 // Supersampled BP (dev_cone_BP_SS / dev_par3D_BP_SS,
@@ -1407,22 +1210,6 @@ bool zc_disabled() {
 }
 
 // z voxels per thread of bp3d_kernel: 16, or 4 / 8 via ASTRA_AMD_BP3D_ZS.
-// ASTRA_AMD_BP3D_LDS=1: the z-constant BP stages detector footprints in LDS
-// (read at every launch)
-bool bp_lds() {
-    const char *e = std::getenv("ASTRA_AMD_BP3D_LDS");
-    return e && e[0] == '1';
-}
-
-// LDS row pitch of the staged BP: ASTRA_AMD_BP3D_LDS_PITCH=<0..15> pads a
-// staged row to that residue modulo 16 quads, -1 (default) to the next odd
-// length (read at every launch)
-int bp_lds_pitch_mod() {
-    const char *e = std::getenv("ASTRA_AMD_BP3D_LDS_PITCH");
-    const int x = e ? std::atoi(e) : -1;
-    return x < 0 ? -1 : (x & 15);
-}
-
 // Measured at 512^3 / 720 x 768^2: 4: 52.7 ms, 8: 50.0, 16: 49.2 per BP
 // launch; at 1024^3 / 1440 x 1536^2 (40-angle chunks) 16 is 1 % faster
 // than 8.
@@ -1648,13 +1435,6 @@ namespace {
 template <int ZS>
 void bp3d_dispatch(int kind, bool zc, const BPArgs &A, hipStream_t s) {
     dim3 grid(((A.nx + 15) / 16) * ((A.ny + 15) / 16), (A.nz + ZS - 1) / ZS);
-    if (zc && bp_lds()) {
-        const int pm = bp_lds_pitch_mod();
-        if (kind == 0) bp3d_lds_kernel<0, ZS><<<grid, 256, 0, s>>>(A, pm);
-        else if (kind == 1) bp3d_lds_kernel<1, ZS><<<grid, 256, 0, s>>>(A, pm);
-        else bp3d_lds_kernel<2, ZS><<<grid, 256, 0, s>>>(A, pm);
-        return;
-    }
     if (kind == 0)
         zc ? bp3d_kernel<0, ZS, true><<<grid, 256, 0, s>>>(A) : bp3d_kernel<0, ZS, false><<<grid, 256, 0, s>>>(A);
     else if (kind == 1)
@@ -1663,12 +1443,51 @@ void bp3d_dispatch(int kind, bool zc, const BPArgs &A, hipStream_t s) {
         zc ? bp3d_kernel<2, ZS, true><<<grid, 256, 0, s>>>(A) : bp3d_kernel<2, ZS, false><<<grid, 256, 0, s>>>(A);
 }
 
-// BP from a row-pair angle-major copy
-void bp3d_run_pairs(const Geom3D &g, const float2 *pairs, float *vol, float out_scale, int kernel,
-                    int mode, const float *upd_w, float lo, float hi, hipStream_t s, unsigned ss) {
+// Supersampling applies
+// to the default cone kernel and to par3d, as in ConeBP_Array / Par3DBP_Array
+// (cuda/3d/cone_bp.cu:351-370, cuda/3d/par3d_bp.cu:285-293).
+bool bp3d_use_ss(const Geom3D &g, int kernel, unsigned ss) {
+    return ss > 1 && (g.kind != ASTRA_AMD_GEOM_CONE || kernel == ASTRA_AMD_KER3D_DEFAULT);
+}
+void bp3d_split_dispatch(int kind, bool zc, const BPArgs &A, hipStream_t s) {
+    const dim3 grid(((A.nx + 7) / 8) * ((A.ny + 7) / 8), (A.nz + kSplitZ - 1) / kSplitZ);
+    if (kind == 0)
+        zc ? bp3d_split_kernel<0, true><<<grid, 256, 0, s>>>(A) : bp3d_split_kernel<0, false><<<grid, 256, 0, s>>>(A);
+    else if (kind == 1)
+        zc ? bp3d_split_kernel<1, true><<<grid, 256, 0, s>>>(A) : bp3d_split_kernel<1, false><<<grid, 256, 0, s>>>(A);
+    else
+        zc ? bp3d_split_kernel<2, true><<<grid, 256, 0, s>>>(A) : bp3d_split_kernel<2, false><<<grid, 256, 0, s>>>(A);
+}
+
+// U and the denominator of the kernel's coefficients are constant along z
+bool bp3d_zc(const Geom3D &g, int kernel) {
+    if (zc_disabled()) return false;
+    if (g.kind == ASTRA_AMD_GEOM_CONE && kernel == ASTRA_AMD_KER3D_FDK_WEIGHTING) return g.zc_fdk;
+    return kernel == ASTRA_AMD_KER3D_2D_WEIGHTING ? g.zc_2d : g.zc_default;
+}
+// Whether a BP runs on the padded single layout of the projections with
+// footprints staged in LDS (bp3d_tile.hip); the others read their row-pair
+// copy.  ASTRA_AMD_BP3D_LDS=0 asks for the gather, 1 for the staged form (read
+// at every launch), ASTRA_AMD_BP3D_ZS, a property of the gather, for the gather.
+// Workgroups of the 16 x 16 column kernels with 16 z voxels per thread.  Below
+// 1024 (4 per CU) the chip is not full: bp3d_split_kernel.
+size_t bp3d_blocks(const Geom3D &g) {
+    return (size_t)((g.nx + 15) / 16) * ((g.ny + 15) / 16) * ((g.nz + 15) / 16);
+}
+constexpr size_t kBpFullBlocks = 1024;
+bool bp3d_use_tiles(const Geom3D &g, int kernel, unsigned ss) {
+    if (g.kind == ASTRA_AMD_GEOM_CYLCONE || bp3d_use_ss(g, kernel, ss) || !bp3d_zc(g, kernel)) return false;
+    const char *e = std::getenv("ASTRA_AMD_BP3D_LDS");
+    if (e && *e) return e[0] != '0';
+    return !std::getenv("ASTRA_AMD_BP3D_ZS") && bp3d_blocks(g) >= kBpFullBlocks;
+}
+
+// BP from the angle-major copy that bp3d_use_tiles names
+void bp3d_run(const Geom3D &g, const float *copy, bool tiles, float *vol, float out_scale, int kernel,
+              int mode, const float *upd_w, float lo, float hi, hipStream_t s, unsigned ss) {
     AMX_REQUIRE(ss >= 1 && ss <= 16, "bp3d: rays per voxel dimension must be in [1, 16]");
     BPArgs A{};
-    A.pp = reinterpret_cast<const float *>(pairs);
+    A.pp = copy;
     A.nu = g.nu; A.nv = g.nv; A.na = g.na;
     A.nx = g.nx; A.ny = g.ny; A.nz = g.nz;
     A.vol = vol;
@@ -1701,39 +1520,19 @@ void bp3d_run_pairs(const Geom3D &g, const float2 *pairs, float *vol, float out_
     const char *pname = g.kind != ASTRA_AMD_GEOM_CONE ? "bp3d_par3d"
                         : (kernel == ASTRA_AMD_KER3D_FDK_WEIGHTING ? "bp3d_fdk" : "bp3d_cone");
     ProfToken pt = prof_begin(pname, (double)g.nx * g.ny * g.nz * g.na, s);
-    int kind;
-    bool zc;
+    int kind = 2;
     if (g.kind == ASTRA_AMD_GEOM_CONE) {
-        if (kernel == ASTRA_AMD_KER3D_FDK_WEIGHTING) {
-            A.ang = g.bp_fdk.as<BP3DAngle>();
-            kind = 0;
-            zc = g.zc_fdk;
-        } else if (kernel == ASTRA_AMD_KER3D_2D_WEIGHTING) {
-            A.ang = g.bp_2d.as<BP3DAngle>();
-            kind = 1;
-            zc = g.zc_2d;
-        } else {
-            A.ang = g.bp_default.as<BP3DAngle>();
-            kind = 0;
-            zc = g.zc_default;
-        }
+        kind = kernel == ASTRA_AMD_KER3D_2D_WEIGHTING ? 1 : 0;
+        A.ang = (kernel == ASTRA_AMD_KER3D_FDK_WEIGHTING  ? g.bp_fdk
+                 : kernel == ASTRA_AMD_KER3D_2D_WEIGHTING ? g.bp_2d
+                                                          : g.bp_default).as<BP3DAngle>();
     } else {
-        if (kernel == ASTRA_AMD_KER3D_2D_WEIGHTING) {
-            A.ang = g.bp_2d.as<BP3DAngle>();
-            A.aw = g.bp_w_2d.as<float>();
-            zc = g.zc_2d;
-        } else {
-            A.ang = g.bp_default.as<BP3DAngle>();
-            A.aw = g.bp_w_default.as<float>();
-            zc = g.zc_default;
-        }
-        kind = 2;
+        const bool w2 = kernel == ASTRA_AMD_KER3D_2D_WEIGHTING;
+        A.ang = (w2 ? g.bp_2d : g.bp_default).as<BP3DAngle>();
+        A.aw = (w2 ? g.bp_w_2d : g.bp_w_default).as<float>();
     }
-    if (zc_disabled()) zc = false;
-    // supersampling applies to the default cone kernel and to par3d, as in
-    // ConeBP_Array / Par3DBP_Array (cuda/3d/cone_bp.cu:351-370,
-    // cuda/3d/par3d_bp.cu:285-293)
-    const bool use_ss = ss > 1 && (g.kind != ASTRA_AMD_GEOM_CONE || kernel == ASTRA_AMD_KER3D_DEFAULT);
+    const bool zc = bp3d_zc(g, kernel);
+    const bool use_ss = bp3d_use_ss(g, kernel, ss);
     if (use_ss) {
         dim3 sgrid(((g.nx + 15) / 16) * ((g.ny + 15) / 16), g.nz);
         if (kind == 0)
@@ -1742,7 +1541,10 @@ void bp3d_run_pairs(const Geom3D &g, const float2 *pairs, float *vol, float out_
             bp3d_ss_kernel<2><<<sgrid, 256, 0, s>>>(A, (int)ss);
     } else {
         const int zs = bp_zs();
-        const size_t plane = (size_t)(A.nv + 2 * kPad) * (A.nu + 2 * kPad) * 2;
+        const char *lds = std::getenv("ASTRA_AMD_BP3D_LDS");
+        const bool split = !tiles && bp3d_blocks(g) < kBpFullBlocks && !(lds && *lds) &&
+                           !std::getenv("ASTRA_AMD_BP3D_ZS");
+        const size_t plane = (size_t)(A.nv + 2 * kPad) * (A.nu + 2 * kPad) * (tiles ? 1 : 2);
         const unsigned na = A.na;
         const unsigned chunk = bp_achunk(plane * na * sizeof(float), na);
         // SET / ADD chunks accumulate in the volume itself; an update mode
@@ -1768,7 +1570,9 @@ void bp3d_run_pairs(const Geom3D &g, const float2 *pairs, float *vol, float out_
                 C.mode = A.mode;
                 C.pre = part ? part->as<float>() : nullptr;
             }
-            if (zs == 4) bp3d_dispatch<4>(kind, zc, C, s);
+            if (tiles) bp3d_tile_launch(kind, C, s);
+            else if (split) bp3d_split_dispatch(kind, zc, C, s);
+            else if (zs == 4) bp3d_dispatch<4>(kind, zc, C, s);
             else if (zs == 16) bp3d_dispatch<16>(kind, zc, C, s);
             else bp3d_dispatch<8>(kind, zc, C, s);
         }
@@ -1782,20 +1586,28 @@ void bp3d_run_pairs(const Geom3D &g, const float2 *pairs, float *vol, float out_
 void bp3d_launch_padded(const Geom3D &g, const float *pp, float *vol, float out_scale, int kernel,
                         int mode, const float *upd_w, float lo, float hi, hipStream_t s,
                         unsigned ss) {
+    if (bp3d_use_tiles(g, kernel, ss)) {
+        bp3d_run(g, pp, true, vol, out_scale, kernel, mode, upd_w, lo, hi, s, ss);
+        return;
+    }
     Scratch pairs(padded_am_elems(g) * sizeof(float2), s);
     am_to_pairs<<<g.na * ((g.nv + 2 * kPad + kPairRows - 1) / kPairRows), 256, 0, s>>>(
         pp, pairs.as<float2>(), g.nu, g.nv);
     AMX_LAUNCHED();
-    bp3d_run_pairs(g, pairs.as<float2>(), vol, out_scale, kernel, mode, upd_w, lo, hi, s, ss);
+    bp3d_run(g, pairs.as<float>(), false, vol, out_scale, kernel, mode, upd_w, lo, hi, s, ss);
 }
 
 void bp3d_launch(const Geom3D &g, const float *proj, float *vol, float out_scale, int kernel,
                  int mode, const float *upd_w, float lo, float hi, hipStream_t s, unsigned ss) {
-    Scratch pairs(padded_am_elems(g) * sizeof(float2), s);
-    proj_to_am_pairs<<<g.na * ((g.nv + 2 * kPad + kPairRows - 1) / kPairRows), 256, 0, s>>>(
-        proj, pairs.as<float2>(), g.nu, g.na, g.nv);
+    const bool tiles = bp3d_use_tiles(g, kernel, ss);
+    Scratch copy(padded_am_elems(g) * (tiles ? sizeof(float) : sizeof(float2)), s);
+    if (tiles)
+        proj_to_padded_am(g, proj, copy.as<float>(), s);
+    else
+        proj_to_am_pairs<<<g.na * ((g.nv + 2 * kPad + kPairRows - 1) / kPairRows), 256, 0, s>>>(
+            proj, copy.as<float2>(), g.nu, g.na, g.nv);
     AMX_LAUNCHED();
-    bp3d_run_pairs(g, pairs.as<float2>(), vol, out_scale, kernel, mode, upd_w, lo, hi, s, ss);
+    bp3d_run(g, copy.as<float>(), tiles, vol, out_scale, kernel, mode, upd_w, lo, hi, s, ss);
 }
 
 // slices per thread of the matched gather (ASTRA_AMD_MATCHED_SLICES:

@@ -148,6 +148,64 @@ __device__ __forceinline__ void fp3d_store(const FPArgs &A, int u, int v, int an
     }
 }
 
+// ------------------------------------------------------------- BP --------
+struct BPArgs {
+    const float *pp;  // padded angle-major projections
+    unsigned nu, nv, na;
+    const BP3DAngle *ang;
+    const float *aw;  // par3d per-angle weights
+    unsigned nx, ny, nz;
+    float osc;
+    float *vol;
+    int mode;
+    const float *uw;  // OUT_UPDATE: per-voxel weights (may be NULL)
+    float lo, hi;     // OUT_UPDATE: clamp
+    const float *pre; // bp3d_kernel: BP of earlier angle chunks, added before the epilogue (or NULL)
+};
+
+// Epilogue of a column of ZS voxels: scale, add the earlier chunks, write
+// in the launch's mode.
+// Every load of the column (earlier chunks, old values, weights) is issued
+// before the first store, so the column's read-modify-write costs one
+// memory round trip, not one per voxel (the compiler cannot reorder a load
+// of vol after a store to vol by itself).  Z0 is the workgroup's, so the
+// bounds tests are uniform.
+template <int ZS>
+__device__ __forceinline__ void bp_column_store(const BPArgs &A, int X, int Y, int Z0,
+                                                const float (&acc)[ZS]) {
+    const int nzr = min(ZS, (int)A.nz - Z0);
+    const size_t plane = (size_t)A.ny * A.nx;
+    const size_t base = ((size_t)Z0 * A.ny + Y) * A.nx + X;
+    const bool old = A.mode != OUT_SET;
+    const bool wts = (A.mode == OUT_EMUPD || A.mode == OUT_UPDATE) && A.uw;
+    float pv[ZS], ov[ZS], wv[ZS];
+#pragma unroll
+    for (int i = 0; i < ZS; ++i) {
+        pv[i] = 0.f;
+        ov[i] = 0.f;
+        wv[i] = 1.f;
+        if (i < nzr) {
+            const size_t idx = base + i * plane;
+            if (A.pre) pv[i] = A.pre[idx];
+            if (old) ov[i] = A.vol[idx];
+            if (wts) wv[i] = A.uw[idx];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < ZS; ++i) {
+        if (i < nzr) {
+            float val = acc[i] * A.osc;
+            if (A.pre) val += pv[i];
+            float out;
+            if (A.mode == OUT_ADD) out = ov[i] + val;
+            else if (A.mode == OUT_SET) out = val;
+            else if (A.mode == OUT_EMUPD) out = ov[i] * (val * wv[i]);
+            else out = fminf(fmaxf(fmaf(wv[i], val, ov[i]), A.lo), A.hi);  // OUT_UPDATE
+            A.vol[base + i * plane] = out;
+        }
+    }
+}
+
 // ------------------------------------------------------------ launch -----
 // Most angles per block of the FP workgroup map (fp_map): an XCD's range
 // is cut into equal blocks of at most this many angles.
@@ -207,5 +265,11 @@ bool adj3d_cols_ok(const Geom3D &g, int grp);
 void adj3d_cols_launch(const Geom3D &g, int grp, const FPArgs &A, const float *proj, const float4 *geo,
                        float4 *q0, float2 *q1, float *yw, float *out, hipStream_t s);
 void adj3d_cols_add(const Geom3D &g, const float *cols, float *vol, hipStream_t s);
+
+// BP with staged detector footprints (bp3d_tile.hip): from the padded single
+// layout, angles [0, A.na), U and the denominator constant along z; `kind` as
+// bp3d_kernel's, kTileZ voxels of a column per thread.
+constexpr int kTileZ = 16;
+void bp3d_tile_launch(int kind, const BPArgs &A, hipStream_t s);
 
 }  // namespace amx
