@@ -164,33 +164,39 @@ __global__ __launch_bounds__(256) void batch_fp_pair(BatchArgs B, const float *_
     }
 }
 
-// The same over 64 detectors x 16 angles per workgroup with the slice rows
-// staged in LDS (fp2d_tile_lds).
+// The same over 64 detectors x 4 kBatchNA angles per workgroup, kBatchNA per
+// wave, with the slice rows staged in LDS (fp2d_wave).
+constexpr int kBatchNA = 4;
 __global__ __launch_bounds__(256) void batch_fp_lds(BatchArgs B, const float *__restrict__ rows,
                                                     const float *__restrict__ cols,
                                                     const float *__restrict__ sinos,
                                                     const float *__restrict__ lw,
                                                     float *__restrict__ out, int mode) {
-    __shared__ Fp2Lds L;
+    constexpr int NA = kBatchNA;
+    __shared__ float buf[4][kFp2Buf];
     const unsigned item = blockIdx.x;
     const unsigned s = find_slice(B.prefix, B.n, item);
     const SliceDesc d = B.desc[s];
     const unsigned local = item - B.prefix[s];
     const unsigned dblocks = (d.nd + 63) / 64;
-    const int det = (local % dblocks) * 64 + (threadIdx.x & 63);
-    const int a0 = (local / dblocks) * 16 + (threadIdx.x >> 6) * kFp2Rays;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int d0 = (local % dblocks) * 64, det = d0 + (threadIdx.x & 63);
+    const int a0 = (local / dblocks) * 4 * NA + wave * NA;
+    if (a0 >= (int)d.na) return;  // uniform over the wave
     const FP2DAngle *fpa = B.fpa + d.ang_off;
     const float *r = rows + d.rows_off, *c = cols + d.cols_off;
-    float val[kFp2Rays];
+    float val[NA];
+    bool mine[NA];
     if (d.kind == ASTRA_AMD_GEOM_FAN)
-        fp2d_tile_lds<true>(det, a0, d.na, d.nd, d.w, d.h, fpa, r, c, val, L);
+        fp2d_wave<true, NA>(d0, a0, d.na, d.nd, 1, d.w, d.h, fpa, r, c, blockIdx.y != 0, val, mine, buf[wave]);
     else
-        fp2d_tile_lds<false>(det, a0, d.na, d.nd, d.w, d.h, fpa, r, c, val, L);
+        fp2d_wave<false, NA>(d0, a0, d.na, d.nd, 1, d.w, d.h, fpa, r, c, blockIdx.y != 0, val, mine, buf[wave]);
     if (det >= (int)d.nd) return;
 #pragma unroll
-    for (int j = 0; j < kFp2Rays; ++j) {
+    for (int j = 0; j < NA; ++j) {
         const int angle = a0 + j;
         if (angle >= (int)d.na) break;
+        if (!mine[j]) continue;
         const size_t oidx = d.psino_off + (size_t)angle * (d.nd + 2 * kPad) + det + kPad;
         if (mode == OUT_SET) {
             out[oidx] = val[j] * d.osc;
@@ -557,7 +563,7 @@ Batch2D *batch2d_build(unsigned n, const int *kinds, const unsigned *ws, const u
             const unsigned rows_per_group = 4 * kBPPY[k];
             acc(b->pre_bp[k], (size_t)((d.w + 63) / 64) * ((d.h + rows_per_group - 1) / rows_per_group));
         }
-        acc(b->pre_fp[3], (size_t)((d.nd + 63) / 64) * ((d.na + 15) / 16));
+        acc(b->pre_fp[3], (size_t)((d.nd + 63) / 64) * ((d.na + 4 * kBatchNA - 1) / (4 * kBatchNA)));
         for (int k = 0; k < 3; ++k) {  // pair tilings: kFPDB[k] dets x 512 / kFPDB[k] angles
             const unsigned db = kFPDB[k], ab = 512 / kFPDB[k];
             acc(b->pre_fp[4 + k], (size_t)((d.nd + db - 1) / db) * ((d.na + ab - 1) / ab));
@@ -637,7 +643,7 @@ void launch_fp(const Batch2D &b, int cfg, const float *sinos, float *out, int mo
     else if (cfg == 2)
         batch_fp<32><<<g, 256, 0, s>>>(a, rows, cols, sinos, lw, out, mode);
     else if (cfg == 3)
-        batch_fp_lds<<<g, 256, 0, s>>>(a, rows, cols, sinos, lw, out, mode);
+        batch_fp_lds<<<dim3(g, 2), 256, 0, s>>>(a, rows, cols, sinos, lw, out, mode);
     else if (cfg == 4)
         batch_fp_pair<64><<<g, 256, 0, s>>>(a, rows, cols, sinos, lw, out, mode);
     else if (cfg == 5)
@@ -649,12 +655,12 @@ void launch_fp(const Batch2D &b, int cfg, const float *sinos, float *out, int mo
 
 // FP candidates: kFPDB tilings (0..2), the LDS-staged one (3) and the
 // kFPDB tilings with two detectors per thread (4..6).  The autotuner times
-// the first three; the others never won on the 4096-slice workload (LDS:
-// no faster; pairs: 197 vs 200 slices/s; workgroups of both kinds in one
-// launch, to keep the texture path and the VALU busy at once: 185) and run
-// by request only.
+// the first four (48 slices of 128 to 1024, per iteration: gathers 3.8 ms,
+// staged 1.4 ms with 4 angles per wave, 1.45 with 3, 1.6 with 2); the
+// pairs never won (197 vs 200 slices/s on 4096 slices) and run by request
+// only.
 constexpr int kFPCandidates = 7;
-constexpr int kFPTimed = 3;
+constexpr int kFPTimed = 4;
 
 // BP candidates: cfg % 3 picks the rows per thread (kBPPY); cfg 0..2 read
 // every tap from global memory, 3..5 from LDS-staged footprints, 6..8 from

@@ -72,6 +72,30 @@ __global__ __launch_bounds__(256) void fp2d_kernel(FP2DArgs A) {
     store_fp(A.out, oidx, val, A.mode, A.rb, idx, A.rw);
 }
 
+// The same with the slice rows staged in LDS (fp2d_wave): 64 detectors x 4 NA
+// angles per group, NA per wave.  Equal to fp2d_kernel's values.
+template <bool FAN, int NA>
+__global__ __launch_bounds__(256, 4) void fp2d_wave_kernel(FP2DArgs A) {
+    __shared__ float buf[4][kFp2Buf];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int d0 = blockIdx.x * 64, det = d0 + (threadIdx.x & 63);
+    const int a0 = (blockIdx.y * 4 + wave) * NA;
+    if (a0 >= (int)A.na) return;  // uniform over the wave
+    float val[NA];
+    bool mine[NA];
+    fp2d_wave<FAN, NA>(d0, a0, A.na, A.nd, A.rays, A.w, A.h, A.ang, A.rows, A.cols, blockIdx.z != 0, val, mine, buf[wave]);
+    if (det >= (int)A.nd) return;
+#pragma unroll
+    for (int j = 0; j < NA; ++j) {
+        const int angle = a0 + j;
+        if (angle >= (int)A.na) break;
+        if (!mine[j]) continue;
+        const size_t idx = (size_t)angle * A.nd + det;
+        const size_t oidx = A.padded_out ? (size_t)angle * (A.nd + 2 * kPad) + det + kPad : idx;
+        store_fp(A.out, oidx, val[j] * A.osc, A.mode, A.rb, idx, A.rw);
+    }
+}
+
 // The same for rays = 1 with two neighbouring detectors per thread
 // (fp2d_value_pair: one 16-byte load per slice serves both rays): 128
 // detectors x 4 angles per group.  Equal to fp2d_kernel's values.
@@ -331,16 +355,45 @@ void fp2d_run(const Geom2D &g, const float *vol, float *sino, float out_scale, i
     if (prof)
         pt = prof_begin(g.kind == ASTRA_AMD_GEOM_FAN ? "fp2d_fan" : "fp2d_par",
                         (double)na_sub * g.nd * rays * std::max(g.w, g.h), s);
+    const bool fan = g.kind == ASTRA_AMD_GEOM_FAN;
     if (rays == 1 && fp2d_pairs()) {
         dim3 pgrid((g.nd + 127) / 128, (na_sub + 3) / 4);
-        if (g.kind == ASTRA_AMD_GEOM_FAN)
+        if (fan)
             fp2d_pair_kernel<true><<<pgrid, 256, 0, s>>>(A);
         else
             fp2d_pair_kernel<false><<<pgrid, 256, 0, s>>>(A);
-    } else if (g.kind == ASTRA_AMD_GEOM_FAN)
-        fp2d_kernel<true><<<grid, 256, 0, s>>>(A);
-    else
-        fp2d_kernel<false><<<grid, 256, 0, s>>>(A);
+    } else if (!fp2d_staged() || (!fan && std::max(g.w, g.h) < 192 && !fp2d_staged_always())) {
+        // few slices per ray: not enough chunks to hide the staging behind.
+        // Gather and staged, parallel: 64^2 / 720 x 96 7.8 and 10.2 us,
+        // 100^2 / 300 x 140 10.2 and 12.0, 200^2 / 100 x 280 20.0 and 18.3;
+        // fan (a division more per gathered ray, both axes in one wave):
+        // 48^2 / 24 x 60 8.9 and 6.6, 100^2 / 300 x 140 15.3 and 11.8
+        if (fan)
+            fp2d_kernel<true><<<grid, 256, 0, s>>>(A);
+        else
+            fp2d_kernel<false><<<grid, 256, 0, s>>>(A);
+    } else {
+        // Angles of a wave share their staged rows; one angle per wave fills
+        // the GPU's 4096 wave slots earlier.  Measured with 1 / 2 / 3 / 4
+        // angles, gather in brackets (us, about 70 of them the call):
+        // 256^2 / 360 x 384 (2160 waves of one angle) 85 / 87 / 96 / 97 (87),
+        // 512^2 / 360 x 768 (4320) 130 / 130 / 138 / 144 (162),
+        // 777^2 / 501 x 1013 (8016) 253 / 198 / 236 / 216 (360),
+        // 1024^2 / 720 x 1536 (17280) 425 / 336 / 331 / 353 (616),
+        // 2048^2 / 1440 x 3072 (69120) 2507 / 1710 / 1574 / 1553 (4146).
+        const size_t blocks = (g.nd + 63) / 64, waves = blocks * na_sub;
+        const unsigned n = waves >= 16384 ? 3 : waves > 4096 ? 2 : 1;
+        const dim3 wgrid((unsigned)blocks, (na_sub + 4 * n - 1) / (4 * n), 2);
+        if (n == 3)
+            fan ? fp2d_wave_kernel<true, 3><<<wgrid, 256, 0, s>>>(A)
+                : fp2d_wave_kernel<false, 3><<<wgrid, 256, 0, s>>>(A);
+        else if (n == 2)
+            fan ? fp2d_wave_kernel<true, 2><<<wgrid, 256, 0, s>>>(A)
+                : fp2d_wave_kernel<false, 2><<<wgrid, 256, 0, s>>>(A);
+        else
+            fan ? fp2d_wave_kernel<true, 1><<<wgrid, 256, 0, s>>>(A)
+                : fp2d_wave_kernel<false, 1><<<wgrid, 256, 0, s>>>(A);
+    }
     AMX_LAUNCHED();
     if (prof) prof_end(pt, s);
 }
@@ -394,6 +447,17 @@ void fp2d_launch_noalloc(const Geom2D &g, const float *vol, float *sino, float o
 // slower: 0.385 vs 0.208 s for the fan 1024^2 SIRT with the row pairs below)
 bool fp2d_pairs() {
     const char *e = std::getenv("ASTRA_AMD_FP2D_PAIRS");
+    return e && e[0] == '1';
+}
+
+// ASTRA_AMD_FP2D_LDS: 0 gathers the taps from global memory, 1 stages slice
+// rows in LDS for every size, unset chooses by size (read at every launch)
+bool fp2d_staged() {
+    const char *e = std::getenv("ASTRA_AMD_FP2D_LDS");
+    return !(e && e[0] == '0');
+}
+bool fp2d_staged_always() {
+    const char *e = std::getenv("ASTRA_AMD_FP2D_LDS");
     return e && e[0] == '1';
 }
 

@@ -280,168 +280,262 @@ __device__ __forceinline__ void bp2d_column(int X, int Y0, unsigned w, unsigned 
 }
 
 // ---- forward projection with slice rows staged in LDS -------------------
-// A workgroup of 256 threads covers 64 detectors x 16 angles: thread t takes
-// detector d0 + (t & 63) at the 4 angles a0 + 4 (t >> 6) + j, j < 4.  When
-// every ray of the group runs along the same axis (rows or columns), the
-// group marches the slices in lockstep, kFp2SC at a time: the interval of
-// padded texels that its rays sample in those slices (bounding interval of
-// each ray's coordinate at the chunk's ends, reduced over the group,
-// widened by one texel) is copied into LDS with coalesced loads, and the
-// samples read LDS.  A chunk whose interval exceeds kFp2Wcap texels, and a
-// group with rays along both axes, sample global memory.  Each ray sums its
-// samples exactly as march2d does (alternating accumulators from its own
-// first slice), so the values equal fp2d_value's.
-constexpr int kFp2SC = 16;     // slices per staged chunk
-constexpr int kFp2Wcap = 256;  // texels per staged slice row
-constexpr int kFp2Rays = 4;    // angles per thread
+// march2d reads the two taps of a sample with one 8-byte gather, which the
+// texture-address path serves at 16 clocks per wave and CU.  Here a wave
+// takes 64 neighbouring detectors at NA neighbouring angles and marches them
+// through the slices together: for a chunk of kFp2SC slices it copies the
+// texels that its rays can sample -- one interval, the same for the chunk's
+// slices -- to LDS with coalesced dword loads (4 clocks each, shared by the NA
+// angles) and takes the taps from there (one read2_b32).  The loads of the
+// next chunk are in flight while this one is sampled; a wave uses its own
+// part of LDS only, in program order: no barrier.
+// At a slice the sample positions of one angle are monotone in the detector
+// (a projective map whose denominator keeps its sign: checked), so those of
+// its first and last lane bound them; the intervals of 64 slices are computed
+// at a time, one per lane.  A chunk whose interval exceeds a staged row takes
+// half the slices and rows of twice the length; one that exceeds those samples
+// global memory.  A wave takes one slice axis: rays of the other one belong to
+// another wave of the launch (both in one wave doubled the longest wave, and
+// with it the launch: 356 -> 300 us in the example below).
+// Every ray adds the samples of march2d in the same order (the slices before
+// and after its own range add exact zeros), so the values equal
+// fp2d_value's.
+// Bound by issue (VALU 10 per sample) and by the second round of waves that
+// does not fill the GPU, no unit saturated.  FP of 1024^2 / 720 x 1536, fan:
+// 719 us with gathers, 276 to 300 here (16 slices per chunk 276, 8: 300).
+constexpr int kFp2SC = 16;      // slices per staged chunk
+constexpr int kFp2Row = 128;    // texels per staged slice row; or half the
+                                // slices and twice the texels
+constexpr int kFp2Buf = kFp2SC * kFp2Row;  // floats per wave
 
-struct Fp2Lds {
-    float buf[kFp2SC * kFp2Wcap];
-    int red[2][2][4];  // [chunk parity][min, max][wave]
-};
+__device__ __forceinline__ int cvt_floor(float x) {  // floor, exact for |x| < 2^31
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
 
-template <bool FAN>
-__device__ __forceinline__ void fp2d_tile_lds(int det, int a0, unsigned na, unsigned nd, unsigned w,
-                                              unsigned h, const FP2DAngle *__restrict__ fpa,
-                                              const float *__restrict__ rows,
-                                              const float *__restrict__ cols, float (&val)[kFp2Rays],
-                                              Fp2Lds &L) {
-    const unsigned tid = threadIdx.x, wave = tid >> 6;
-    Ray2D R[kFp2Rays];
-    bool on[kFp2Rays];
-    int vert = 0, horiz = 0;
+// Samples of SC slices from LDS rows of ROW texels.  CLIP: some sample is
+// outside the padded row.
+template <int NA, int SC, int ROW, bool CLIP>
+__device__ __forceinline__ void fp2d_chunk(const Ray2D (&R)[NA], float sf, float hi_t, unsigned at,
+                                           float (&acc)[NA][2]) {
+    typedef const __attribute__((address_space(3))) float *lptr;
+    constexpr int G = 8;  // samples whose taps are in flight
 #pragma unroll
-    for (int j = 0; j < kFp2Rays; ++j) {
-        const int angle = a0 + j;
-        on[j] = det < (int)nd && angle < (int)na;
-        R[j].a = 0.f;
-        R[j].c = 0.5f;
-        R[j].scale = 0.f;
-        R[j].lo = 1;
-        R[j].hi = 0;
-        val[j] = 0.f;
-        if (on[j]) {
-            const FP2DAngle &G = fpa[angle];
-            const bool v = ray_vertical<FAN>(G, det);
-            R[j] = ray2d<FAN>(G, det + 0.5, v, w, h);
-            vert |= v ? 1 : 0;
-            horiz |= v ? 0 : 1;
+    for (int g = 0; g < SC * NA; g += G) {
+        float t0[G], t1[G], wt[G];
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            const int i = (g + e) / NA, j = (g + e) % NA;
+            float t = fmaf(R[j].a, sf + (float)i, R[j].c);
+            if (CLIP) t = clamp_pad(t, hi_t);
+            const lptr q = (lptr)(size_t)(((unsigned)t << 2) + (at + i * (ROW * 4)));
+            t0[e] = q[0];
+            t1[e] = q[1];
+            wt[e] = frac(t);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            const int i = (g + e) / NA, j = (g + e) % NA;
+            acc[j][i & 1] += lerp(t0[e], t1[e], wt[e]);
         }
     }
-    const __amdgpu_buffer_rsrc_t rr = texel_rsrc(rows), rc = texel_rsrc(cols);
-    const bool any_v = __syncthreads_or(vert), any_h = __syncthreads_or(horiz);
-    if (any_v && any_h) {
-        // rays along both axes: each ray from global memory
+}
+
+// Values of detectors d0 + lane at angles a0 .. a0 + NA - 1 (clamped to the last
+// ones), `rays` sub-rays each, of the rays that run along the rows (V) or the
+// columns: `mine`; buf: kFp2Buf floats of LDS of this wave.
+template <bool FAN, int NA>
+__device__ __forceinline__ void fp2d_wave(int d0, int a0, unsigned na, unsigned nd, unsigned rays,
+                                          unsigned w, unsigned h, const FP2DAngle *__restrict__ fpa,
+                                          const float *__restrict__ rows, const float *__restrict__ cols,
+                                          bool V, float (&val)[NA], bool (&mine)[NA], float *buf) {
+    const int lane = threadIdx.x & 63;
+    const int det = min(d0 + lane, (int)nd - 1);
+    const unsigned lds = (unsigned)(size_t)(__attribute__((address_space(3))) float *)buf;
 #pragma unroll
-        for (int j = 0; j < kFp2Rays; ++j) {
-            if (!on[j]) continue;
-            const bool v = ray_vertical<FAN>(fpa[a0 + j], det);
-            const float s = v ? march2d(rr, w + 2 * kPad, (float)w + 2.5f, R[j])
-                              : march2d(rc, h + 2 * kPad, (float)h + 2.5f, R[j]);
-            val[j] = s * R[j].scale;
-        }
-        return;
+    for (int j = 0; j < NA; ++j) val[j] = 0.f;
+    bool any = false;
+    unsigned long long m[NA];
+#pragma unroll
+    for (int j = 0; j < NA; ++j) {
+        mine[j] = ray_vertical<FAN>(fpa[min(a0 + j, (int)na - 1)], det) == V;
+        m[j] = __ballot(mine[j]);
+        any = any || m[j];
     }
-    if (!any_v && !any_h) return;  // no ray in the group
-    const bool V = any_v;
-    const float *base = V ? rows : cols;
-    const unsigned pitch = V ? w + 2 * kPad : h + 2 * kPad;
-    const float hi_t = V ? (float)w + 2.5f : (float)h + 2.5f;
-    // slice range of the group
-    int lo = 1 << 30, hi = -1;
+    if (!any) return;
+#pragma unroll 1
+    for (unsigned k = 0; k < rays; ++k) {
+        const double fdet = det + (0.5 + k) / (double)rays;
+        Ray2D R[NA];
+        const unsigned pitch = (V ? w : h) + 2 * kPad, nsl = V ? h : w;
+        bool simple = (unsigned long long)pitch * nsl < (1ull << 29);  // 32-bit byte offsets
+        const float hi_t = (float)(V ? w : h) + 2.5f;
+        int glo = 1 << 30, ghi = -1;
 #pragma unroll
-    for (int j = 0; j < kFp2Rays; ++j)
-        if (on[j] && R[j].lo <= R[j].hi) {
-            lo = min(lo, R[j].lo);
-            hi = max(hi, R[j].hi);
-        }
-    lo = wave_min(lo);
-    hi = wave_max(hi);
-    if ((tid & 63) == 0) {
-        L.red[1][0][wave] = lo;
-        L.red[1][1][wave] = hi;
-    }
-    __syncthreads();
-    int glo = L.red[1][0][0], ghi = L.red[1][1][0];
-#pragma unroll
-    for (int k = 1; k < 4; ++k) {
-        glo = min(glo, L.red[1][0][k]);
-        ghi = max(ghi, L.red[1][1][k]);
-    }
-    float acc0[kFp2Rays], acc1[kFp2Rays];
-#pragma unroll
-    for (int j = 0; j < kFp2Rays; ++j) acc0[j] = acc1[j] = 0.f;
-    int parity = 0;
-    for (int cs = glo; cs <= ghi; cs += kFp2SC, parity ^= 1) {
-        const int ce = min(cs + kFp2SC - 1, ghi);
-        // interval of texels sampled in slices [cs, ce]
-        int tlo = 1 << 30, thi = -1;
-#pragma unroll
-        for (int j = 0; j < kFp2Rays; ++j) {
-            const int sb = max(cs, R[j].lo), se = min(ce, R[j].hi);
-            if (on[j] && sb <= se) {
-                const float tb = clamp_pad(fmaf(R[j].a, (float)sb, R[j].c), hi_t);
-                const float te = clamp_pad(fmaf(R[j].a, (float)se, R[j].c), hi_t);
-                tlo = min(tlo, (int)fminf(tb, te));
-                thi = max(thi, (int)fmaxf(tb, te));
+        for (int j = 0; j < NA; ++j) {
+            const FP2DAngle &G = fpa[min(a0 + j, (int)na - 1)];
+            R[j] = ray2d<FAN>(G, fdet, V, w, h);
+            if (mine[j] && R[j].lo <= R[j].hi) {
+                glo = min(glo, R[j].lo);
+                ghi = max(ghi, R[j].hi);
+            }
+            if (FAN && m[j]) {
+                const double den = G.r[V] - G.p0[V] - (fdet - 0.5) * G.u[V];
+                const unsigned long long neg = __ballot(mine[j] && den < 0.0);
+                const int first = __builtin_ctzll(m[j]), last = 63 - __builtin_clzll(m[j]);
+                simple = simple && (neg == 0 || neg == m[j]) && __builtin_popcountll(m[j]) == last - first + 1;
+                // the other lanes follow the nearest one
+                const int near = min(max(lane, first), last);
+                R[j].a = __shfl(R[j].a, near, 64);
+                R[j].c = __shfl(R[j].c, near, 64);
             }
         }
-        tlo = wave_min(tlo);
-        thi = wave_max(thi);
-        // L.red[parity] was last read before the previous chunk's second
-        // barrier
-        if ((tid & 63) == 0) {
-            L.red[parity][0][wave] = tlo;
-            L.red[parity][1][wave] = thi;
-        }
-        __syncthreads();  // also: every thread is done with the previous chunk's rows
-        int t0 = L.red[parity][0][0], t1 = L.red[parity][1][0];
+        if (!simple) {
+            const __amdgpu_buffer_rsrc_t rg = texel_rsrc(V ? rows : cols);
 #pragma unroll
-        for (int k = 1; k < 4; ++k) {
-            t0 = min(t0, L.red[parity][0][k]);
-            t1 = max(t1, L.red[parity][1][k]);
+            for (int j = 0; j < NA; ++j)
+                if (mine[j])
+                    val[j] += march2d(rg, pitch, hi_t, R[j]) * R[j].scale;
+            continue;
         }
-        t0 = max(0, t0 - 1);
-        t1 = min((int)pitch - 1, t1 + 2);
-        const int wd = t1 - t0 + 1;
-        const bool staged = t1 >= t0 && wd <= kFp2Wcap;
-        if (staged) {
-            const int nrows = ce - cs + 1;
-            for (int i = (int)tid; i < nrows * kFp2Wcap; i += 256) {
-                const int r = i / kFp2Wcap, c = i & (kFp2Wcap - 1);
-                if (c < wd) L.buf[i] = base[(size_t)(cs + r) * pitch + t0 + c];
-            }
-        }
-        __syncthreads();
-        for (int sl = cs; sl <= ce; ++sl) {
-            const float sf = (float)sl;
-            const float *lrow = L.buf + (sl - cs) * kFp2Wcap;
-            const float *grow = base + (size_t)sl * pitch;
+        glo = __builtin_amdgcn_readfirstlane(wave_min(glo));
+        ghi = __builtin_amdgcn_readfirstlane(wave_max(ghi));
+        if (glo > ghi) continue;  // val += 0
+        // an angle without rays in this pass follows one that has some
 #pragma unroll
-            for (int j = 0; j < kFp2Rays; ++j) {
-                if (!on[j] || sl < R[j].lo || sl > R[j].hi) continue;
-                const float t = clamp_pad(fmaf(R[j].a, sf, R[j].c), hi_t);
-                const float f = floorf(t);
-                float2 q;
-                if (staged) {
-                    // inside the staged interval by its margin; the clamp
-                    // only keeps the LDS address inside the row
-                    const int o = min(max((int)f - t0, 0), kFp2Wcap - 2);
-                    q = make_float2(lrow[o], lrow[o + 1]);
-                } else {
-                    q = ld2b(grow, (unsigned)f << 2);
+        for (int j = 0; j < NA; ++j) {
+            if (m[j]) continue;
+#pragma unroll
+            for (int i = 0; i < NA; ++i)
+                if (m[i]) {
+                    R[j].a = R[i].a;
+                    R[j].c = R[i].c;
                 }
-                const float x = lerp(q.x, q.y, t - f);
-                if ((sl - R[j].lo) & 1)
-                    acc1[j] += x;
-                else
-                    acc0[j] += x;
-            }
         }
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(first_lane_ptr(V ? rows : cols)), (short)0, (int)(nsl * pitch * 4u), 0x00020000);
+
+        int plo = 0, phi = 0, pclip = 0, pbase = 0;
+        auto params = [&](int s0) {
+            pbase = s0;
+            const float sf = (float)(s0 + lane);
+            float tmin = INFINITY, tmax = -INFINITY;
+#pragma unroll
+            for (int j = 0; j < NA; ++j) {
+                const float tf = fmaf(lane_value(R[j].a, 0), sf, lane_value(R[j].c, 0));
+                const float tl = fmaf(lane_value(R[j].a, 63), sf, lane_value(R[j].c, 63));
+                tmin = fminf(tmin, fminf(tf, tl));
+                tmax = fmaxf(tmax, fmaxf(tf, tl));
+            }
+            // 0.01: far beyond the rounding of the rays in between
+            pclip = (tmin < 0.51f || tmax > hi_t - 0.01f) ? 1 : 0;
+            plo = cvt_floor(clamp_pad(tmin - 0.01f, hi_t));
+            phi = cvt_floor(clamp_pad(tmax + 0.01f, hi_t)) + 1;
+        };
+        // chunk in flight: first texel, texels, slices, clamping
+        float g[2 * kFp2SC];
+        int zb = 0, len = 0, cs = 0, clip = 0;
+        auto issue = [&](int s) {
+            if (s + kFp2SC - pbase > 64) params(s);
+            const int q = s - pbase;
+            // positions are linear in the slice: the ends of the chunk bound it
+            const int l0 = __builtin_amdgcn_readlane(plo, q), h0 = __builtin_amdgcn_readlane(phi, q);
+            const int c0 = __builtin_amdgcn_readlane(pclip, q);
+            cs = kFp2SC;
+            zb = min(l0, __builtin_amdgcn_readlane(plo, q + kFp2SC - 1));
+            len = max(h0, __builtin_amdgcn_readlane(phi, q + kFp2SC - 1)) - zb + 1;
+            clip = c0 | __builtin_amdgcn_readlane(pclip, q + kFp2SC - 1);
+            if (len > kFp2Row) {
+                cs = kFp2SC / 2;
+                zb = min(l0, __builtin_amdgcn_readlane(plo, q + kFp2SC / 2 - 1));
+                len = max(h0, __builtin_amdgcn_readlane(phi, q + kFp2SC / 2 - 1)) - zb + 1;
+                clip = c0 | __builtin_amdgcn_readlane(pclip, q + kFp2SC / 2 - 1);
+                if (len > 2 * kFp2Row) return;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    if (b > 1 && len <= 64 * b) break;
+                    const int off = (zb + lane + 64 * b) * 4;
+#pragma unroll
+                    for (int i = 0; i < kFp2SC / 2; ++i)
+                        g[b * (kFp2SC / 2) + i] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            rs, off, min(s + i, (int)nsl - 1) * (int)(pitch * 4u), 0));
+                }
+                return;
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                if (b > 0 && len <= 64 * b) break;
+                const int off = (zb + lane + 64 * b) * 4;
+#pragma unroll
+                for (int i = 0; i < kFp2SC; ++i)
+                    g[b * kFp2SC + i] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                        rs, off, min(s + i, (int)nsl - 1) * (int)(pitch * 4u), 0));
+            }
+        };
+        float acc[NA][2];
+#pragma unroll
+        for (int j = 0; j < NA; ++j) acc[j][0] = acc[j][1] = 0.f;
+        params(glo);
+        issue(glo);
+        for (int s = glo; s <= ghi;) {
+            const int cz = zb, cn = len, cc = clip, step = cs;
+            const int left = (int)nsl - s;
+            if (step == kFp2SC) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    if (b > 0 && cn <= 64 * b) break;
+                    if (left >= kFp2SC) {
+#pragma unroll
+                        for (int i = 0; i < kFp2SC; ++i) buf[i * kFp2Row + 64 * b + lane] = g[b * kFp2SC + i];
+                    } else {  // slices past the last one: zeros
+#pragma unroll
+                        for (int i = 0; i < kFp2SC; ++i)
+                            buf[i * kFp2Row + 64 * b + lane] = i < left ? g[b * kFp2SC + i] : 0.f;
+                    }
+                }
+            } else if (cn <= 2 * kFp2Row) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    if (b > 1 && cn <= 64 * b) break;
+#pragma unroll
+                    for (int i = 0; i < kFp2SC / 2; ++i)
+                        buf[i * (2 * kFp2Row) + 64 * b + lane] = i < left ? g[b * (kFp2SC / 2) + i] : 0.f;
+                }
+            }
+            if (s + step <= ghi) issue(s + step);
+            const unsigned at = __builtin_amdgcn_readfirstlane(lds - 4u * (unsigned)cz);
+            if (step == kFp2SC) {
+                if (cc)
+                    fp2d_chunk<NA, kFp2SC, kFp2Row, true>(R, (float)s, hi_t, at, acc);
+                else
+                    fp2d_chunk<NA, kFp2SC, kFp2Row, false>(R, (float)s, hi_t, at, acc);
+            } else if (cn <= 2 * kFp2Row) {
+                fp2d_chunk<NA, kFp2SC / 2, 2 * kFp2Row, true>(R, (float)s, hi_t, at, acc);
+            } else {
+                for (int i = 0; i < step && s + i <= ghi; ++i) {
+#pragma unroll
+                    for (int j = 0; j < NA; ++j) {
+                        const float t = clamp_pad(fmaf(R[j].a, (float)(s + i), R[j].c), hi_t);
+                        const float2 q = ld2b(V ? rows : cols, ((unsigned)(s + i) * pitch + (unsigned)t) << 2);
+                        const float x = lerp(q.x, q.y, frac(t));
+                        if (i & 1) acc[j][1] += x;
+                        else acc[j][0] += x;
+                    }
+                }
+            }
+            s += step;
+        }
+#pragma unroll
+        for (int j = 0; j < NA; ++j)
+            if (mine[j]) val[j] += (acc[j][0] + acc[j][1]) * R[j].scale;
     }
 #pragma unroll
-    for (int j = 0; j < kFp2Rays; ++j)
-        if (on[j]) val[j] = (acc0[j] + acc1[j]) * R[j].scale;
+    for (int j = 0; j < NA; ++j) val[j] /= (float)rays;
 }
 
 // ---- back projection with sinogram footprints staged in LDS -------------
