@@ -234,30 +234,33 @@ __global__ __launch_bounds__(256) void batch_bp(BatchArgs B, const float *__rest
                       mode, pw, lo, hi);
 }
 
-// The same with the sinogram footprints staged in LDS (bp2d_tile_lds).
+// The same with the sinogram footprints staged in LDS (bp2d_wave).
 template <int PY>
 __global__ __launch_bounds__(256) void batch_bp_lds(BatchArgs B, const float *__restrict__ psino,
                                                     const float *__restrict__ pw,
                                                     float *__restrict__ vols, int mode, float lo,
                                                     float hi) {
-    __shared__ Bp2Lds L;
+    __shared__ float buf[4][kBp2Buf];
     const unsigned item = blockIdx.x;
     const unsigned s = find_slice(B.prefix, B.n, item);
     const SliceDesc d = B.desc[s];
     const unsigned local = item - B.prefix[s];
     const unsigned xblocks = (d.w + 63) / 64;
     const int X0 = (local % xblocks) * 64;
-    const int Yt0 = (local / xblocks) * 4 * PY;
-    float acc[PY];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int X = X0 + (threadIdx.x & 63);
+    const int Y0 = ((local / xblocks) * 4 + wave) * PY;
+    if (Y0 >= (int)d.h) return;
+    float col[PY][1], acc[PY];
     const float *sp = psino + d.psino_off;
     const BP2DAngle *ang = B.bpa + d.ang_off;
     if (d.kind == ASTRA_AMD_GEOM_FAN)
-        bp2d_tile_lds<1, PY>(X0, Yt0, d.w, d.h, d.na, d.nd, sp, ang, acc, L);
+        bp2d_wave<1, 64, 1, PY>(X0, Y0, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, buf[wave]);
     else
-        bp2d_tile_lds<0, PY>(X0, Yt0, d.w, d.h, d.na, d.nd, sp, ang, acc, L);
-    const int X = X0 + (threadIdx.x & 63);
-    const int Y0 = Yt0 + (threadIdx.x >> 6) * PY;
-    if (X >= (int)d.w || Y0 >= (int)d.h) return;
+        bp2d_wave<0, 64, 1, PY>(X0, Y0, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, buf[wave]);
+    if (X >= (int)d.w) return;
+#pragma unroll
+    for (int i = 0; i < PY; ++i) acc[i] = col[i][0];
     store_bp_rows<PY>(vols, d.vol_off + (size_t)Y0 * d.w + X, d.w, min(PY, (int)d.h - Y0), acc, d.osc,
                       mode, pw, lo, hi);
 }
@@ -321,7 +324,7 @@ __host__ __device__ __forceinline__ unsigned persist_units(unsigned h, unsigned 
 
 union PersistLds {
     float tile[64][65];
-    Bp2Lds bp;
+    float bp[4][kBp2Buf];
 };
 
 // WPE: the fewest waves per SIMD the register allocation must allow (1: no
@@ -428,10 +431,16 @@ batch_sirt_persistent(PersistArgs P) {
                 const int Y0 = Yt0 + (tid >> 6) * PY;
                 float acc[PY];
                 if (LDS) {
+                    const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+                    const int Yw = Yt0 + (int)wave * PY;
+                    if (Yw >= (int)d.h) continue;
+                    float col[PY][1];
                     if (d.kind == ASTRA_AMD_GEOM_FAN)
-                        bp2d_tile_lds<1, PY>(X0, Yt0, d.w, d.h, d.na, d.nd, sp, ang, acc, S.bp);
+                        bp2d_wave<1, 64, 1, PY>(X0, Yw, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, S.bp[wave]);
                     else
-                        bp2d_tile_lds<0, PY>(X0, Yt0, d.w, d.h, d.na, d.nd, sp, ang, acc, S.bp);
+                        bp2d_wave<0, 64, 1, PY>(X0, Yw, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, S.bp[wave]);
+#pragma unroll
+                    for (int i = 0; i < PY; ++i) acc[i] = col[i][0];
                 }
                 if (X >= (int)d.w || Y0 >= (int)d.h) continue;
                 if (!LDS) {
@@ -665,7 +674,9 @@ constexpr int kFPTimed = 4;
 // BP candidates: cfg % 3 picks the rows per thread (kBPPY); cfg 0..2 read
 // every tap from global memory, 3..5 from LDS-staged footprints, 6..8 from
 // global memory two rows per load.  The autotuner times 0..5 (the row
-// pairs never won: 175 vs 173 slices/s at best).
+// pairs never won: 175 vs 173 slices/s at best).  48 slices of 128 to 1024,
+// per iteration: gathers 2.35 ms, staged 1.45 ms with 8 rows, 1.8 with 4;
+// tiles of 32 x 16 pixels per wave 1.42, not worth a form of their own.
 constexpr int kBPCandidates = 9;
 constexpr int kBPTimed = 6;
 

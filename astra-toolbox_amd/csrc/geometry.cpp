@@ -439,6 +439,20 @@ Geom2D *geom2d_build(int kind, unsigned w, unsigned h, unsigned na, unsigned nd,
     auto *g = new Geom2D();
     g->kind = kind;
     g->w = w; g->h = h; g->na = na; g->nd = nd;
+    g->bp_reach = 0.f;
+    for (const BP2DAngle &b : bp) {
+        double dmin = INFINITY, dmax = -INFINITY, r = 0.0;
+        for (int j = 0; j < 4; ++j) {
+            const double x = (j & 1 ? 0.5 : -0.5) * w, y = (j & 2 ? 0.5 : -0.5) * h;
+            const double den = b.den[0] + x * b.den[1] + y * b.den[2];
+            const double t = (b.num[0] + x * b.num[1] + y * b.num[2]) / den;
+            dmin = std::min(dmin, den);
+            dmax = std::max(dmax, den);
+            r = std::max(r, (std::fabs(b.num[1] - t * b.den[1]) + std::fabs(b.num[2] - t * b.den[2])) / std::fabs(den));
+        }
+        if (!(dmin > 0.0 || dmax < 0.0)) r = INFINITY;
+        g->bp_reach = std::max(g->bp_reach, (float)r);
+    }
     g->vecs.assign(vecs, vecs + 6 * (size_t)na);
     try {
         AMX_HIP(hipGetDevice(&g->device));

@@ -195,6 +195,9 @@ struct Geom2D {
     std::vector<float> vecs;  // 6 per angle
     DevArray fp;              // FP2DAngle[na]
     DevArray bp, bp_fbp;      // BP2DAngle[na]
+    // bound of |dt/dx| + |dt/dy|, texels of a row per pixel, over the slice's
+    // corners and the angles; infinite where a source lies inside the slice
+    float bp_reach;
     // FBP state built on first use: the default Ram-Lak filter, the fan
     // pre-weights [nd] and short-scan Parker weights [na][nd]
     mutable std::mutex fbp_mu;
@@ -247,7 +250,7 @@ void fp2d_launch(const Geom2D &g, const float *vol, float *sino, float out_scale
 void fp2d_launch_range(const Geom2D &g, const float *vol, float *sino, float out_scale, int mode,
                        const float *resid_b, const float *resid_w, bool padded_out, unsigned rays,
                        unsigned a0, unsigned na_sub, hipStream_t s);
-bool bp2d_lds();
+int bp2d_lds();
 bool fp2d_pairs();
 bool fp2d_staged();
 bool fp2d_staged_always();

@@ -140,20 +140,52 @@ __global__ __launch_bounds__(256) void bp2d_kernel(BP2DArgs A) {
                       A.uw, A.lo, A.hi);
 }
 
-// The same with the sinogram footprints staged in LDS (bp2d_tile_lds):
-// equal floats, taps from LDS instead of the texture-address path.
+// The same with the sinogram footprints staged in LDS (bp2d_wave): equal
+// floats, taps from LDS instead of the texture-address path.
 template <int KIND>
 __global__ __launch_bounds__(256) void bp2d_lds_kernel(BP2DArgs A) {
     constexpr int PY = 4;
-    __shared__ Bp2Lds L;
-    const int X0 = blockIdx.x * 64, Yt0 = blockIdx.y * 4 * PY;
-    float acc[PY];
-    bp2d_tile_lds<KIND, PY>(X0, Yt0, A.w, A.h, A.na, A.nd, A.sp, A.ang, acc, L);
-    const int X = X0 + (threadIdx.x & 63);
-    const int Y0 = Yt0 + (threadIdx.x >> 6) * PY;
-    if (X >= (int)A.w || Y0 >= (int)A.h) return;
+    __shared__ float buf[4][kBp2Buf];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int X0 = blockIdx.x * 64, X = X0 + (threadIdx.x & 63);
+    const int Y0 = (blockIdx.y * 4 + wave) * PY;
+    if (Y0 >= (int)A.h) return;
+    float col[PY][1], acc[PY];
+    bp2d_wave<KIND, 64, 1, PY>(X0, Y0, A.w, A.h, 0, A.na, A.na, A.nd, A.sp, A.ang, col, buf[wave]);
+    if (X >= (int)A.w) return;
+#pragma unroll
+    for (int i = 0; i < PY; ++i) acc[i] = col[i][0];
     store_bp_rows<PY>(A.vol, (size_t)Y0 * A.w + X, A.w, min(PY, (int)A.h - Y0), acc, A.osc, A.mode,
                       A.uw, A.lo, A.hi);
+}
+
+// 8 TX x 8 TY pixels per group, the angles split over its NW waves (bp2d_wave),
+// the waves' sums added in their order.  A 256^2 slice has 64 of
+// bp2d_kernel's groups, each with a serial chain of loads over all angles: 69
+// us at 180 angles, 9 here with 16 x 16 pixels and 16 waves.
+template <int KIND, int TX, int TY, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void bp2d_tile_kernel(BP2DArgs A) {
+    constexpr int N = TX * TY;
+    constexpr int kBuf = kBp2Buf > 64 * N ? kBp2Buf : 64 * N;
+    __shared__ float buf[NW][kBuf];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int X0 = blockIdx.x * 8 * TX, Y0 = blockIdx.y * 8 * TY;
+    float acc[TY][TX];
+    bp2d_wave<KIND, 8, TX, TY>(X0, Y0, A.w, A.h, (unsigned)((size_t)A.na * wave / NW),
+                               (unsigned)((size_t)A.na * (wave + 1) / NW), A.na, A.nd, A.sp, A.ang, acc, buf[wave]);
+#pragma unroll
+    for (int j = 0; j < TY; ++j)
+#pragma unroll
+        for (int i = 0; i < TX; ++i) buf[wave][(j * TX + i) * 64 + lane] = acc[j][i];
+    __syncthreads();
+    for (int p = wave; p < N; p += NW) {
+        float sum[1] = {buf[0][p * 64 + lane]};
+#pragma unroll
+        for (int k = 1; k < NW; ++k) sum[0] += buf[k][p * 64 + lane];
+        const int X = X0 + (int)(lane & 7) + 8 * (p % TX), Y = Y0 + (int)(lane >> 3) + 8 * (p / TX);
+        if (X < (int)A.w && Y < (int)A.h)
+            store_bp_rows<1>(A.vol, (size_t)Y * A.w + X, A.w, 1, sum, A.osc, A.mode, A.uw, A.lo, A.hi);
+    }
 }
 
 // Supersampled BP (devBP_SS / devFanBP_SS, cuda/2d/par_bp.cu:90-137,
@@ -469,11 +501,12 @@ bool bp2d_pairs() {
     return e && e[0] == '1';
 }
 
-// ASTRA_AMD_BP2D_LDS=1 takes the taps of the 2D BP from LDS-staged
-// footprints instead of global memory (read at every launch)
-bool bp2d_lds() {
+// ASTRA_AMD_BP2D_LDS: 0 gathers the taps of the 2D BP from global memory, 1
+// takes them from LDS-staged rows with the gather's floats, unset (-1)
+// chooses tiles by size (read at every launch)
+int bp2d_lds() {
     const char *e = std::getenv("ASTRA_AMD_BP2D_LDS");
-    return e && e[0] == '1';
+    return e && *e ? e[0] == '1' : -1;
 }
 
 void bp2d_launch_padded(const Geom2D &g, const float *sp, float *vol, float out_scale, bool fbp,
@@ -503,7 +536,38 @@ void bp2d_launch_padded(const Geom2D &g, const float *sp, float *vol, float out_
         const int kind = g.kind == ASTRA_AMD_GEOM_PAR ? 0 : (fbp ? 2 : 1);
         A.ang = (kind == 2 ? g.bp_fbp : g.bp).as<BP2DAngle>();
         const bool pr = bp2d_pairs();
-        if (bp2d_lds()) {
+        const int lds = bp2d_lds();
+        // Tiles of 32 x 32 / 32 x 16 / 16 x 16 pixels with the angles split
+        // over 4 / 8 / 16 waves, while the longest footprint fits a staged
+        // row.  Measured (us, about 65 of them the call; gather in brackets):
+        // parallel 256^2 / 180 x 384 85 / 69 / 65 (122), 384^2 / 360 x 512
+        // 113 / 89 / 86 (187), 512^2 / 360 x 768 112 / 89 / 94 (184),
+        // 1024^2 / 720 x 1536 240 / 241 / 308 (381), 2048^2 / 1440 x 3072
+        // 1245 / 1369 / 1926 (2903); fan 1024^2 344 / 319 / 365 (403).
+        const size_t tiles = (size_t)((g.w + 31) / 32) * ((g.h + 15) / 16);
+        const float reach = g.bp_reach;
+        // A few angles are not worth a wave's set-up: 1024^2 / 1 angle 4.2 us
+        // gathered, 7.2 in tiles, / 24 angles (parallel) 15.2 and 13.0, (fan)
+        // 15.2 and 16.4; 512^2 / 24 11.8 and 6.3.
+        const bool few = g.na < 8 || (tiles >= 2048 && g.na < (kind == 0 ? 16u : 32u));
+        if (lds < 0 && !std::getenv("ASTRA_AMD_BP2D_PAIRS") && !few && 15.f * reach <= kBp2Row - 6) {
+            if (tiles < 512 || 31.f * reach > kBp2Row - 6) {
+                dim3 tg((g.w + 15) / 16, (g.h + 15) / 16);
+                if (kind == 0) bp2d_tile_kernel<0, 2, 2, 16><<<tg, 1024, 0, s>>>(A);
+                else if (kind == 1) bp2d_tile_kernel<1, 2, 2, 16><<<tg, 1024, 0, s>>>(A);
+                else bp2d_tile_kernel<2, 2, 2, 16><<<tg, 1024, 0, s>>>(A);
+            } else if (tiles < 8192) {
+                dim3 tg((g.w + 31) / 32, (g.h + 15) / 16);
+                if (kind == 0) bp2d_tile_kernel<0, 4, 2, 8><<<tg, 512, 0, s>>>(A);
+                else if (kind == 1) bp2d_tile_kernel<1, 4, 2, 8><<<tg, 512, 0, s>>>(A);
+                else bp2d_tile_kernel<2, 4, 2, 8><<<tg, 512, 0, s>>>(A);
+            } else {
+                dim3 tg((g.w + 31) / 32, (g.h + 31) / 32);
+                if (kind == 0) bp2d_tile_kernel<0, 4, 4, 4><<<tg, 256, 0, s>>>(A);
+                else if (kind == 1) bp2d_tile_kernel<1, 4, 4, 4><<<tg, 256, 0, s>>>(A);
+                else bp2d_tile_kernel<2, 4, 4, 4><<<tg, 256, 0, s>>>(A);
+            }
+        } else if (lds == 1) {
             if (kind == 0) bp2d_lds_kernel<0><<<grid, 256, 0, s>>>(A);
             else if (kind == 1) bp2d_lds_kernel<1><<<grid, 256, 0, s>>>(A);
             else bp2d_lds_kernel<2><<<grid, 256, 0, s>>>(A);

@@ -539,29 +539,38 @@ __device__ __forceinline__ void fp2d_wave(int d0, int a0, unsigned na, unsigned 
 }
 
 // ---- back projection with sinogram footprints staged in LDS -------------
-// A workgroup of 256 threads covers 64 columns x (4 PY) rows (thread: column
-// X0 + (tid & 63), rows Y0 + (tid >> 6) PY ..).  For every block of kBp2KA
-// angles, the texels of each angle's sinogram row that the tile's taps can
-// reach are copied into LDS with coalesced loads, and the taps read LDS.
+// bp2d_column reads the two taps of an update with one 8-byte gather (16
+// clocks per wave and CU).  Here a wave covers a tile of LX TX x (64 / LX) TY
+// pixels -- lane l its pixels (l % LX + LX i, l / LX + 64 / LX j) -- and
+// copies, kBp2KA angles at a time, the texels of each angle's sinogram row
+// that the tile's taps can reach to its own part of LDS with coalesced loads;
+// the taps are then read from there (one read2_b32).  The loads of the next
+// angles are in flight while these are summed, and nothing is shared between
+// waves: no barrier.
 // The reach is the bounding interval of the tap coordinate at the tile's
 // four corner pixels (t is linear-fractional in the pixel position, so its
 // extremes over the tile are at the corners, and the clamp is monotone),
 // widened by one texel on each side, far beyond the fp32 rounding of the
-// taps' incremental coordinates.  An angle whose interval exceeds
-// kBp2Wcap texels, or whose denominator changes sign over the tile, is
-// sampled from global memory.  Taps, weights and the order of the sums are
+// taps' incremental coordinates; 64 angles' intervals are computed at a
+// time, one per lane.  An angle whose interval exceeds kBp2Row texels, or
+// whose denominator changes sign over the tile, is sampled from global memory.
+// Lanes in 8 x 8 squares: the footprint is short for the updates it serves,
+// and the taps of neighbouring lanes share LDS words.
+// Bound by the VALU (parallel 7, fan 11 instructions per update, the fan's
+// reciprocal at a quarter of the rate): BP of 1024^2 / 720 x 1536 338 -> 225
+// us (fan, 10.7 clocks per update and CU), of 777 x 641 / 501 x 1013 209 ->
+// 79 us (parallel, 5.6).
+// With LX = 64 and TX = 1 the taps, weights and the order of the sums are
 // those of bp2d_column, so both give the same floats.
-constexpr int kBp2KA = 16;     // angles per staged block
-constexpr int kBp2Wcap = 256;  // texels per staged angle row (power of two)
+constexpr int kBp2KA = 4;     // angles per staged block
+constexpr int kBp2Row = 256;  // texels per staged angle row
+constexpr int kBp2Buf = kBp2KA * kBp2Row;  // floats per wave
 
-struct Bp2Lds {
-    float buf[kBp2KA * kBp2Wcap];
-    int2 fp[kBp2KA];  // (first texel, width); width 0: from global memory
-};
-
+// Interval of an angle packed in an int: first texel | texels << 20 |
+// no tap is clamped << 30; texels 0: from global memory.
 template <int KIND>
-__device__ __forceinline__ int2 bp2d_footprint(const BP2DAngle &c, float fx0, float fx1, float fy0,
-                                               float fy1, float hi, int pitch) {
+__device__ __forceinline__ int bp2d_footprint(const BP2DAngle &c, float fx0, float fx1, float fy0,
+                                              float fy1, float hi, int pitch) {
     float tmin = INFINITY, tmax = -INFINITY, dmin = INFINITY, dmax = -INFINITY;
     for (int j = 0; j < 4; ++j) {
         const float fx = (j & 1) ? fx1 : fx0, fy = (j & 2) ? fy1 : fy0;
@@ -569,93 +578,158 @@ __device__ __forceinline__ int2 bp2d_footprint(const BP2DAngle &c, float fx0, fl
         const float den = fmaf(fy, c.den[2], fmaf(fx, c.den[1], c.den[0]));
         dmin = fminf(dmin, den);
         dmax = fmaxf(dmax, den);
-        const float fr = (KIND == 0 || KIND == 3) ? 1.f : 1.f / den;
-        const float t = clamp_pad(num * fr, hi);
+        const float t = num * ((KIND == 0 || KIND == 3) ? 1.f : 1.f / den);
         tmin = fminf(tmin, t);
         tmax = fmaxf(tmax, t);
     }
     const bool sign_ok = KIND == 0 || KIND == 3 || dmin > 0.f || dmax < 0.f;
-    if (!sign_ok || !__builtin_isfinite(tmin) || !__builtin_isfinite(tmax)) return make_int2(0, 0);
+    if (!sign_ok || !__builtin_isfinite(tmin) || !__builtin_isfinite(tmax)) return 0;
+    const bool inner = tmin >= 1.5f && tmax <= hi - 1.f;
     // taps read texels floor(t) and floor(t) + 1 (t >= 0.5 after the clamp)
-    const int t0 = max(0, (int)tmin - 1), t1 = min(pitch - 1, (int)tmax + 2);
+    const int t0 = max(0, (int)clamp_pad(tmin, hi) - 1);
+    const int t1 = min(pitch - 1, (int)clamp_pad(tmax, hi) + 2);
     const int wd = t1 - t0 + 1;
-    return wd <= kBp2Wcap ? make_int2(t0, wd) : make_int2(0, 0);
+    return wd <= kBp2Row && t0 < (1 << 20) ? t0 | wd << 20 | (inner ? 1 << 30 : 0) : 0;
 }
 
-template <int KIND, int PY>
-__device__ __forceinline__ void bp2d_tile_lds(int X0, int Yt0, unsigned w, unsigned h, unsigned na,
-                                              unsigned nd, const float *__restrict__ sp,
-                                              const BP2DAngle *__restrict__ ang, float *acc,
-                                              Bp2Lds &L) {
-    const unsigned tid = threadIdx.x;
-    const int X = X0 + (int)(tid & 63);
-    const int Y0 = Yt0 + (int)(tid >> 6) * PY;
-    const bool active = X < (int)w && Y0 < (int)h;
-    const float fx = X - 0.5f * w + 0.5f;
-    const float fy0 = -(Y0 - 0.5f * h + 0.5f);  // world y of row Y0
-    // tile corners (pixels inside the slice)
+// One angle's updates of a wave's tile; at: LDS byte address of texel 0 of
+// the angle's row (LDS), or the row's byte offset in rs.
+template <int KIND, int LX, int TX, int TY, bool CLIP, bool LDS>
+__device__ __forceinline__ void bp2d_angle(const BP2DAngle &c, float fx, float fy, float hi, unsigned at,
+                                           __amdgpu_buffer_rsrc_t rs, float (&acc)[TY][TX]) {
+    typedef const __attribute__((address_space(3))) float *lptr;
+    constexpr bool PAR = KIND == 0 || KIND == 3;
+    constexpr int N = TX * TY, G = N < 8 ? N : 8;  // updates whose taps are in flight
+    constexpr float sx = LX, sy = 64 / LX;
+    // steps and weight in vector registers (an operand in a scalar one
+    // halves the rate of an addition)
+    float nx = sx * c.num[1], ny = sy * c.num[2], dx = sx * c.den[1], dy = sy * c.den[2], cw = c.w;
+    asm("" : "+v"(nx), "+v"(ny), "+v"(dx), "+v"(dy), "+v"(cw));
+    float nrow = fmaf(fy, c.num[2], fmaf(fx, c.num[1], c.num[0]));
+    float drow = fmaf(fy, c.den[2], fmaf(fx, c.den[1], c.den[0]));
+    float num = nrow, den = drow;
+#pragma unroll
+    for (int g = 0; g < N; g += G) {
+        float q0[G], q1[G], wt[G], wg[G];
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            const float fr = PAR ? 1.f : __builtin_amdgcn_rcpf(den);
+            float t = PAR ? num : num * fr;
+            if (CLIP) t = clamp_pad(t, hi);
+            if (LDS) {
+                const lptr q = (lptr)(size_t)(((unsigned)t << 2) + at);
+                q0[e] = q[0];
+                q1[e] = q[1];
+            } else {
+                const int o = (int)(((unsigned)t << 2) + at);
+                q0[e] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0));
+                q1[e] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, o + 4, 0, 0));
+            }
+            wt[e] = frac(t);
+            wg[e] = KIND == 0 ? cw : KIND == 1 ? fr : KIND == 2 ? fr * fr : 1.f;
+            if ((g + e + 1) % TX == 0) {  // next row: world y decreases
+                nrow -= ny;
+                drow -= dy;
+                num = nrow;
+                den = drow;
+            } else {
+                num += nx;
+                den += dx;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            float &a = acc[(g + e) / TX][(g + e) % TX];
+            a = fmaf(wg[e], lerp(q0[e], q1[e], wt[e]), a);
+        }
+    }
+}
+
+// Sums over the angles [alo, ahi) of the pixels of the tile at (X0, Y0), a
+// wave's own; buf: kBp2Buf floats of LDS of this wave.
+template <int KIND, int LX, int TX, int TY>
+__device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h, unsigned alo, unsigned ahi,
+                                          unsigned na, unsigned nd, const float *__restrict__ sp,
+                                          const BP2DAngle *__restrict__ ang, float (&acc)[TY][TX],
+                                          float *buf) {
+    typedef const __attribute__((address_space(4))) float *cptr;  // scalar loads
+    const int lane = threadIdx.x & 63;
+    const unsigned lds = (unsigned)(size_t)(__attribute__((address_space(3))) float *)buf;
+    const float fx = (X0 + lane % LX) - 0.5f * w + 0.5f;
+    const float fy = -((Y0 + lane / LX) - 0.5f * h + 0.5f);  // world y
+    // corner pixels of the tile inside the slice
     const float cx0 = X0 - 0.5f * w + 0.5f;
-    const float cx1 = min(X0 + 63, (int)w - 1) - 0.5f * w + 0.5f;
-    const float cy0 = -(Yt0 - 0.5f * h + 0.5f);
-    const float cy1 = -(min(Yt0 + 4 * PY - 1, (int)h - 1) - 0.5f * h + 0.5f);
+    const float cx1 = min(X0 + LX * TX - 1, (int)w - 1) - 0.5f * w + 0.5f;
+    const float cy0 = -(Y0 - 0.5f * h + 0.5f);
+    const float cy1 = -(min(Y0 + 64 / LX * TY - 1, (int)h - 1) - 0.5f * h + 0.5f);
     const unsigned pitch = nd + 2 * kPad;
     const float hi = (float)nd + 2.5f;
-    const __amdgpu_buffer_rsrc_t rs = texel_rsrc(sp);  // unstaged angles
+    // rows a .. a + kBp2KA - 1, as far as they exist
+    auto rows = [&](unsigned a) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(first_lane_ptr(sp + (size_t)a * pitch)), (short)0,
+                                                 (int)(min((unsigned)kBp2KA, na - a) * pitch * 4u), 0x00020000);
+    };
 #pragma unroll
-    for (int i = 0; i < PY; ++i) acc[i] = 0.f;
-    for (unsigned a0 = 0; a0 < na; a0 += kBp2KA) {
-        __syncthreads();  // the previous block's rows are no longer read
-        if (tid < (unsigned)kBp2KA)
-            L.fp[tid] = (a0 + tid < na) ? bp2d_footprint<KIND>(ang[a0 + tid], cx0, cx1, cy0, cy1,
-                                                               hi, (int)pitch)
-                                        : make_int2(0, 0);
-        __syncthreads();
-#pragma unroll 4
-        for (int i = (int)tid; i < kBp2KA * kBp2Wcap; i += 256) {
-            const int k = i / kBp2Wcap, j = i & (kBp2Wcap - 1);
-            const int2 f = L.fp[k];
-            if (j < f.y) L.buf[i] = sp[(size_t)(a0 + k) * pitch + f.x + j];
-        }
-        __syncthreads();
-        if (!active) continue;
-        const unsigned nk = min((unsigned)kBp2KA, na - a0);
-        for (unsigned k = 0; k < nk; ++k) {
-            const BP2DAngle c = ang[a0 + k];
-            // the footprint is the same for every lane: keep it in scalar
-            // registers (a scalar branch, and the LDS row offset folded
-            // into the tap's address computation)
-            const int fx0 = __builtin_amdgcn_readfirstlane(L.fp[k].x);
-            const int fwd = __builtin_amdgcn_readfirstlane(L.fp[k].y);
-            float num = fmaf(fy0, c.num[2], fmaf(fx, c.num[1], c.num[0]));
-            float den = fmaf(fy0, c.den[2], fmaf(fx, c.den[1], c.den[0]));
-            const unsigned rowi = (a0 + k) * pitch;  // first texel of the row
-            // LDS byte offset of texel 0 of the row: a tap's address is
-            // one shift-and-add of its texel index
-            const unsigned lb = __builtin_amdgcn_readfirstlane((unsigned)((int)k * kBp2Wcap - fx0) * 4u);
+    for (int j = 0; j < TY; ++j)
 #pragma unroll
-            for (int i = 0; i < PY; ++i) {
-                float fr = (KIND == 0 || KIND == 3) ? 1.f : __builtin_amdgcn_rcpf(den);
-                float t = clamp_pad(num * fr, hi);
-                const int ti = (int)t;  // t >= 0.5: truncation is the floor
-                float2 q;
-                if (fwd) {
-                    // texels ti, ti + 1 lie inside the staged interval
-                    // [fx0, fx0 + fwd - 1]: the footprint widens the taps'
-                    // range by a texel on each side, far beyond the rounding
-                    // between its corner coordinates and the taps'
-                    // incremental ones (the tests replay both on the host)
-                    const float *l = reinterpret_cast<const float *>(
-                        reinterpret_cast<const char *>(L.buf) + (lb + ((unsigned)ti << 2)));
-                    q = make_float2(l[0], l[1]);
-                } else {
-                    q = ld2i(rs, rowi + (unsigned)ti);
-                }
-                float val = lerp(q.x, q.y, frac(t));
-                float wgt = (KIND == 0) ? c.w : (KIND == 1 ? fr : (KIND == 2 ? fr * fr : 1.f));
-                acc[i] = fmaf(wgt, val, acc[i]);
-                num -= c.num[2];
-                den -= c.den[2];
+        for (int i = 0; i < TX; ++i) acc[j][i] = 0.f;
+    if (alo >= ahi) return;
+
+    int pk = 0;
+    int in[kBp2KA];  // intervals of the angles in flight
+    float g[kBp2KA][kBp2Row / 64];
+    auto issue = [&](unsigned a) {
+        const unsigned q = (a - alo) & 63;
+        const __amdgpu_buffer_rsrc_t rs = rows(a);
+        if (q == 0)
+            pk = bp2d_footprint<KIND>(ang[min(a + lane, na - 1)], cx0, cx1, cy0, cy1, hi, (int)pitch);
+#pragma unroll
+        for (int k = 0; k < kBp2KA; ++k) {
+            in[k] = __builtin_amdgcn_readlane(pk, q + k);
+            const int off = ((in[k] & 0xfffff) + lane) * 4;
+            const int row = (int)(min((unsigned)k, na - 1 - a) * pitch * 4u), wd = (in[k] >> 20) & 0x3ff;
+#pragma unroll
+            for (int b = 0; b < kBp2Row / 64; ++b) {
+                if (b > 0 && wd <= 64 * b) break;
+                g[k][b] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off + 256 * b, row, 0));
             }
+        }
+    };
+    issue(alo);
+    for (unsigned a = alo; a < ahi; a += kBp2KA) {
+        int cur[kBp2KA];
+#pragma unroll
+        for (int k = 0; k < kBp2KA; ++k) {
+            cur[k] = in[k];
+            const int wd = (cur[k] >> 20) & 0x3ff;
+#pragma unroll
+            for (int b = 0; b < kBp2Row / 64; ++b) {
+                if (b > 0 && wd <= 64 * b) break;
+                buf[k * kBp2Row + 64 * b + lane] = g[k][b];
+            }
+        }
+        if (a + kBp2KA < ahi) issue(a + kBp2KA);
+        const __amdgpu_buffer_rsrc_t rs = rows(a);  // unstaged angles
+#pragma unroll 1
+        for (unsigned k = 0; k < min((unsigned)kBp2KA, ahi - a); ++k) {
+            int f = cur[0];
+#pragma unroll
+            for (int i = 1; i < kBp2KA; ++i) f = k == i ? cur[i] : f;
+            const cptr cp = (cptr)(size_t)first_lane_ptr(reinterpret_cast<const float *>(ang + a + k));
+            BP2DAngle c;
+            for (int i = 0; i < 3; ++i) {
+                c.num[i] = cp[i];
+                c.den[i] = cp[3 + i];
+            }
+            c.w = cp[6];
+            const unsigned at = __builtin_amdgcn_readfirstlane(lds + k * (kBp2Row * 4) - 4u * (f & 0xfffff));
+            if (f >> 30)
+                bp2d_angle<KIND, LX, TX, TY, false, true>(c, fx, fy, hi, at, rs, acc);
+            else if (f >> 20)
+                bp2d_angle<KIND, LX, TX, TY, true, true>(c, fx, fy, hi, at, rs, acc);
+            else
+                bp2d_angle<KIND, LX, TX, TY, true, false>(c, fx, fy, hi, k * pitch * 4u, rs, acc);
         }
     }
 }
