@@ -7,6 +7,7 @@ unchunked job execution of CCompositeGeometryManager
 (src/CompositeGeometryManager.cpp:1115-1280).  Device memory and streams come
 from torch; all arithmetic runs in libastra_amd.
 """
+import contextlib
 import ctypes
 import threading
 
@@ -49,7 +50,7 @@ def gpu_memory_limit():
 
 
 def device(index=None):
-    if torch is None or not torch.cuda.is_available():
+    if torch is None or not (torch.cuda.is_initialized() or torch.cuda.is_available()):
         raise AstraError("no GPU available: the ASTRA GPU path needs a ROCm device")
     i = _default_gpu[0] if index is None else int(index)
     if i >= torch.cuda.device_count():
@@ -57,12 +58,23 @@ def device(index=None):
     return torch.device("cuda", i)
 
 
+_current = contextlib.nullcontext()
+
+
+def on_gpu(dev):
+    """Context with `dev` as the current device (none to enter when it is)."""
+    return _current if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
+# torch.cuda.current_stream builds a Stream object (5 us a call, the raw
+# handle 0.3); a small projection is a few such calls long.
 def stream_ptr(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(dev.index))
 
 
 def sync(dev):
-    torch.cuda.current_stream(dev).synchronize()
+    with on_gpu(dev):  # the default stream's handle names the current device's
+        _lib.call("astra_amd_stream_sync", stream_ptr(dev))
 
 
 def ptr(t):
@@ -198,7 +210,7 @@ def fp(proj, vol_t, proj_t, mode=_lib.MODE_SET, scale=1.0):
     _check_tensor(vol_t, proj.vol_shape, "volume")
     _check_tensor(proj_t, proj.proj_shape, "projection data")
     h = ctypes.c_void_p(proj.handle(dev))
-    with torch.cuda.device(dev):
+    with on_gpu(dev):
         s = stream_ptr(dev)
         if proj.is3d:
             p = proj.params3d(scale)
@@ -214,7 +226,7 @@ def bp(proj, proj_t, vol_t, mode=_lib.MODE_SET, scale=1.0, kernel=None, fbp_weig
     _check_tensor(vol_t, proj.vol_shape, "volume")
     _check_tensor(proj_t, proj.proj_shape, "projection data")
     h = ctypes.c_void_p(proj.handle(dev))
-    with torch.cuda.device(dev):
+    with on_gpu(dev):
         s = stream_ptr(dev)
         if proj.is3d:
             p = proj.params3d(scale, kernel)
@@ -391,7 +403,14 @@ def link_data(kind, geom, shape, obj):
     if isinstance(obj, np.ndarray) and not obj.flags.writeable:
         raise ValueError("Failed to link dlpack array: read-only arrays are not supported")
     try:
-        t = torch.from_dlpack(obj)
+        if type(obj) is torch.Tensor and obj.layout == torch.strided and not obj.requires_grad \
+                and obj.device.type in ("cpu", "cuda") and not (obj.is_conj() or obj.is_neg()):
+            # what the exchange below gives for a plain tensor (the same
+            # storage, a version counter of its own), without its 15 us
+            t = obj.data
+            t.data_ptr()  # a transform's wrapper has none: refused, as there
+        else:
+            t = torch.from_dlpack(obj)
     except Exception as e:  # noqa: BLE001 - map producer errors to ValueError
         raise ValueError("Failed to link dlpack array: %s" % e)
     if t.dtype != torch.float32:

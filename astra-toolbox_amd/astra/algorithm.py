@@ -249,7 +249,7 @@ class FBP_CUDA(_Algo):
         s = self.sino.on_device(dev).clone()
         v = self.vol.on_device(dev, init=False)
         h = ctypes.c_void_p(self.proj.handle(dev))
-        with torch.cuda.device(dev):
+        with _core.on_gpu(dev):
             f = _cached_filter(self._filters, dev, self.proj.proj_shape[1], self.proj.proj_shape[0],
                                self.filter)
             _lib.call("astra_amd_fbp2d", h, _core.ptr(s), _core.ptr(v), scale, self.short_scan,
@@ -277,7 +277,7 @@ class FDK_CUDA(_Algo):
     def run(self, iterations=1, mode=_lib.MODE_SET):
         nv, na, nu = self.proj.proj_shape
         dev = self.proj.device()
-        with torch.cuda.device(dev):
+        with _core.on_gpu(dev):
             f = _cached_filter(self._filters, dev, nu, na, self.filter)
         composite.fdk(self.proj, self.sino, self.vol, mode, f, self.short_scan)
 
