@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "lib", "obj")
 OUT = os.path.join(HERE, "lib", "libastra_amd.so")
-SOURCES = ["geometry.cpp", "proj3d.hip", "fp3d_cols.hip", "adj3d_cols.hip", "bp3d_tile.hip", "proj2d.hip", "filter.hip", "arith.hip",
+SOURCES = ["geometry.cpp", "proj3d.hip", "fp3d_cols.hip", "adj3d_cols.hip", "bp3d_tile.hip", "bp3d_flat.hip", "proj2d.hip", "filter.hip", "arith.hip",
            "algorithms.cpp", "batch2d.hip", "profiling.cpp", "calib.hip", "capi.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("ASTRA_AMD_ARCH", "gfx950")

@@ -255,9 +255,9 @@ __global__ __launch_bounds__(256) void batch_bp_lds(BatchArgs B, const float *__
     const float *sp = psino + d.psino_off;
     const BP2DAngle *ang = B.bpa + d.ang_off;
     if (d.kind == ASTRA_AMD_GEOM_FAN)
-        bp2d_wave<1, 64, 1, PY>(X0, Y0, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, buf[wave]);
+        bp2d_wave<1, 64, 1, PY>(X0, Y0, d.w, d.h, 0, d.na, d.na, d.nd, d.nd + 2 * kPad, sp, ang, col, buf[wave]);
     else
-        bp2d_wave<0, 64, 1, PY>(X0, Y0, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, buf[wave]);
+        bp2d_wave<0, 64, 1, PY>(X0, Y0, d.w, d.h, 0, d.na, d.na, d.nd, d.nd + 2 * kPad, sp, ang, col, buf[wave]);
     if (X >= (int)d.w) return;
 #pragma unroll
     for (int i = 0; i < PY; ++i) acc[i] = col[i][0];
@@ -436,9 +436,9 @@ batch_sirt_persistent(PersistArgs P) {
                     if (Yw >= (int)d.h) continue;
                     float col[PY][1];
                     if (d.kind == ASTRA_AMD_GEOM_FAN)
-                        bp2d_wave<1, 64, 1, PY>(X0, Yw, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, S.bp[wave]);
+                        bp2d_wave<1, 64, 1, PY>(X0, Yw, d.w, d.h, 0, d.na, d.na, d.nd, d.nd + 2 * kPad, sp, ang, col, S.bp[wave]);
                     else
-                        bp2d_wave<0, 64, 1, PY>(X0, Yw, d.w, d.h, 0, d.na, d.na, d.nd, sp, ang, col, S.bp[wave]);
+                        bp2d_wave<0, 64, 1, PY>(X0, Yw, d.w, d.h, 0, d.na, d.na, d.nd, d.nd + 2 * kPad, sp, ang, col, S.bp[wave]);
 #pragma unroll
                     for (int i = 0; i < PY; ++i) acc[i] = col[i][0];
                 }

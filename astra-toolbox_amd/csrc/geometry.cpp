@@ -390,7 +390,30 @@ Geom3D *geom3d_build(int kind, unsigned nx, unsigned ny, unsigned nz, unsigned n
     g->zc_fdk = !cyl && zconst(bf);
     g->zc_2d = !cyl && zconst(b2);
     for (int k = 0; k < 3; ++k) g->cols[k] = cols_bound(*g, k);
+    // (a difference below the rounding of a row's coordinate is none)
+    g->flat = kind == ASTRA_AMD_GEOM_PAR3D && g->zc_default && g->zc_2d;
+    const double eps = std::ldexp(1.0, -24) * std::max(nv, 64u);
+    std::vector<BP2DAngle> fd(na), f2(na);
+    for (unsigned a = 0; a < na && g->flat; ++a) {
+        const float *v = bd[a].nv, *v0 = bd[0].nv;
+        const float *u = bd[a].nu;
+        g->flat = std::fabs(v[0]) * nx / 2.0 <= eps && std::fabs(v[1]) * ny / 2.0 <= eps &&
+                  std::fabs((double)v[2] - v0[2]) * nz / 2.0 + std::fabs((double)v[3] - v0[3]) <= eps;
+        // rows of a 2D slice run towards -y
+        fd[a] = BP2DAngle{{u[3], u[0], -u[1]}, {1.f, 0.f, 0.f}, wd[a], 0.f};
+        f2[a] = BP2DAngle{{b2[a].nu[3], b2[a].nu[0], -b2[a].nu[1]}, {1.f, 0.f, 0.f}, w2[a], 0.f};
+        g->flat_reach = std::max({g->flat_reach, std::fabs(u[0]) + std::fabs(u[1]),
+                                  std::fabs(b2[a].nu[0]) + std::fabs(b2[a].nu[1])});
+    }
+    g->flat_v[0] = bd[0].nv[2];
+    g->flat_v[1] = bd[0].nv[3];
     try {
+        if (g->flat) {
+            g->bp_flat_default = DevArray(sizeof(BP2DAngle) * na);
+            g->bp_flat_default.upload(fd.data(), sizeof(BP2DAngle) * na);
+            g->bp_flat_2d = DevArray(sizeof(BP2DAngle) * na);
+            g->bp_flat_2d.upload(f2.data(), sizeof(BP2DAngle) * na);
+        }
         g->fp = DevArray(sizeof(FP3DAngle) * na);
         g->fp.upload(g->fp_host.data(), sizeof(FP3DAngle) * na);
         g->bp_default = DevArray(sizeof(BP3DAngle) * na);

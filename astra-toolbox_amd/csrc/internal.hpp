@@ -180,6 +180,13 @@ struct Geom3D {
     // detector), so the BP hoists them out of its z loop
     bool zc_default = false, zc_fdk = false, zc_2d = false;
     ColsBound cols[3];
+    // par3d with horizontal rays and a vertical detector, the same rows at
+    // every angle: the BP is a 2D BP of each detector row and an
+    // interpolation at row flat_v[0] * z + flat_v[1] (z from the centre,
+    // padded rows).  Coefficients per weight set; reach as bp_reach
+    bool flat = false;
+    float flat_v[2], flat_reach = 0.f;
+    DevArray bp_flat_default, bp_flat_2d;  // BP2DAngle[na]
     DevArray group_idx[3];               // int[dir_count[k]] angle lists
     // FDK pre-weights [nv][nu] and default Ram-Lak filter, built on first use
     mutable std::mutex fdk_mu;

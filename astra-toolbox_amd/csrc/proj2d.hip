@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void bp2d_lds_kernel(BP2DArgs A) {
     const int Y0 = (blockIdx.y * 4 + wave) * PY;
     if (Y0 >= (int)A.h) return;
     float col[PY][1], acc[PY];
-    bp2d_wave<KIND, 64, 1, PY>(X0, Y0, A.w, A.h, 0, A.na, A.na, A.nd, A.sp, A.ang, col, buf[wave]);
+    bp2d_wave<KIND, 64, 1, PY>(X0, Y0, A.w, A.h, 0, A.na, A.na, A.nd, A.nd + 2 * kPad, A.sp, A.ang, col, buf[wave]);
     if (X >= (int)A.w) return;
 #pragma unroll
     for (int i = 0; i < PY; ++i) acc[i] = col[i][0];
@@ -159,33 +159,18 @@ __global__ __launch_bounds__(256) void bp2d_lds_kernel(BP2DArgs A) {
                       A.uw, A.lo, A.hi);
 }
 
-// 8 TX x 8 TY pixels per group, the angles split over its NW waves (bp2d_wave),
-// the waves' sums added in their order.  A 256^2 slice has 64 of
+// 8 TX x 8 TY pixels per group, the angles split over its NW waves.  A 256^2 slice has 64 of
 // bp2d_kernel's groups, each with a serial chain of loads over all angles: 69
 // us at 180 angles, 9 here with 16 x 16 pixels and 16 waves.
 template <int KIND, int TX, int TY, int NW>
 __global__ __launch_bounds__(64 * NW, 4) void bp2d_tile_kernel(BP2DArgs A) {
-    constexpr int N = TX * TY;
-    constexpr int kBuf = kBp2Buf > 64 * N ? kBp2Buf : 64 * N;
-    __shared__ float buf[NW][kBuf];
-    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int X0 = blockIdx.x * 8 * TX, Y0 = blockIdx.y * 8 * TY;
-    float acc[TY][TX];
-    bp2d_wave<KIND, 8, TX, TY>(X0, Y0, A.w, A.h, (unsigned)((size_t)A.na * wave / NW),
-                               (unsigned)((size_t)A.na * (wave + 1) / NW), A.na, A.nd, A.sp, A.ang, acc, buf[wave]);
-#pragma unroll
-    for (int j = 0; j < TY; ++j)
-#pragma unroll
-        for (int i = 0; i < TX; ++i) buf[wave][(j * TX + i) * 64 + lane] = acc[j][i];
-    __syncthreads();
-    for (int p = wave; p < N; p += NW) {
-        float sum[1] = {buf[0][p * 64 + lane]};
-#pragma unroll
-        for (int k = 1; k < NW; ++k) sum[0] += buf[k][p * 64 + lane];
-        const int X = X0 + (int)(lane & 7) + 8 * (p % TX), Y = Y0 + (int)(lane >> 3) + 8 * (p / TX);
-        if (X < (int)A.w && Y < (int)A.h)
-            store_bp_rows<1>(A.vol, (size_t)Y * A.w + X, A.w, 1, sum, A.osc, A.mode, A.uw, A.lo, A.hi);
-    }
+    __shared__ float buf[NW][kBp2TileBuf<TX, TY>];
+    bp2d_tile<KIND, TX, TY, NW>(blockIdx.x * 8 * TX, blockIdx.y * 8 * TY, A.w, A.h, A.na, A.nd, A.nd + 2 * kPad, A.sp,
+                                A.ang, buf, [&](int X, int Y, float sum) {
+                                    const float out[1] = {sum};
+                                    store_bp_rows<1>(A.vol, (size_t)Y * A.w + X, A.w, 1, out, A.osc, A.mode, A.uw,
+                                                     A.lo, A.hi);
+                                });
 }
 
 // Supersampled BP (devBP_SS / devFanBP_SS, cuda/2d/par_bp.cu:90-137,

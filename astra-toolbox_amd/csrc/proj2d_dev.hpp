@@ -647,10 +647,12 @@ __device__ __forceinline__ void bp2d_angle(const BP2DAngle &c, float fx, float f
 }
 
 // Sums over the angles [alo, ahi) of the pixels of the tile at (X0, Y0), a
-// wave's own; buf: kBp2Buf floats of LDS of this wave.
+// wave's own; buf: kBp2Buf floats of LDS of this wave.  Angle a's padded row
+// starts at sp[a * stride]; kBp2KA strides fit in 32-bit byte offsets.
 template <int KIND, int LX, int TX, int TY>
 __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h, unsigned alo, unsigned ahi,
-                                          unsigned na, unsigned nd, const float *__restrict__ sp,
+                                          unsigned na, unsigned nd, size_t stride,
+                                          const float *__restrict__ sp,
                                           const BP2DAngle *__restrict__ ang, float (&acc)[TY][TX],
                                           float *buf) {
     typedef const __attribute__((address_space(4))) float *cptr;  // scalar loads
@@ -665,10 +667,12 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
     const float cy1 = -(min(Y0 + 64 / LX * TY - 1, (int)h - 1) - 0.5f * h + 0.5f);
     const unsigned pitch = nd + 2 * kPad;
     const float hi = (float)nd + 2.5f;
+    const unsigned step = (unsigned)stride * 4u;
     // rows a .. a + kBp2KA - 1, as far as they exist
     auto rows = [&](unsigned a) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(first_lane_ptr(sp + (size_t)a * pitch)), (short)0,
-                                                 (int)(min((unsigned)kBp2KA, na - a) * pitch * 4u), 0x00020000);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(first_lane_ptr(sp + a * stride)), (short)0,
+                                                 (int)((min((unsigned)kBp2KA, na - a) - 1) * step + pitch * 4u),
+                                                 0x00020000);
     };
 #pragma unroll
     for (int j = 0; j < TY; ++j)
@@ -688,7 +692,7 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
         for (int k = 0; k < kBp2KA; ++k) {
             in[k] = __builtin_amdgcn_readlane(pk, q + k);
             const int off = ((in[k] & 0xfffff) + lane) * 4;
-            const int row = (int)(min((unsigned)k, na - 1 - a) * pitch * 4u), wd = (in[k] >> 20) & 0x3ff;
+            const int row = (int)(min((unsigned)k, na - 1 - a) * step), wd = (in[k] >> 20) & 0x3ff;
 #pragma unroll
             for (int b = 0; b < kBp2Row / 64; ++b) {
                 if (b > 0 && wd <= 64 * b) break;
@@ -729,7 +733,7 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
             else if (f >> 20)
                 bp2d_angle<KIND, LX, TX, TY, true, true>(c, fx, fy, hi, at, rs, acc);
             else
-                bp2d_angle<KIND, LX, TX, TY, true, false>(c, fx, fy, hi, k * pitch * 4u, rs, acc);
+                bp2d_angle<KIND, LX, TX, TY, true, false>(c, fx, fy, hi, k * step, rs, acc);
         }
     }
 }
@@ -805,6 +809,35 @@ __device__ __forceinline__ void vol2d_copy_tile(const float *__restrict__ vol,
         int pc = c0 + i, pr = r0 + tx;
         int c = pc - kPad;
         if (c >= 0 && c < (int)w && pr < ph) cols[(size_t)c * ph + pr] = tile[tx][i];
+    }
+}
+
+// 8 TX x 8 TY pixels of a group of NW waves, each wave the sums over its part
+// of the angles; store(X, Y, sum): the waves' sums added in their order.
+template <int TX, int TY>
+constexpr int kBp2TileBuf = kBp2Buf > 64 * TX * TY ? kBp2Buf : 64 * TX * TY;
+
+template <int KIND, int TX, int TY, int NW, class F>
+__device__ __forceinline__ void bp2d_tile(int X0, int Y0, unsigned w, unsigned h, unsigned na, unsigned nd,
+                                          size_t stride, const float *__restrict__ sp,
+                                          const BP2DAngle *__restrict__ ang,
+                                          float (&buf)[NW][kBp2TileBuf<TX, TY>], F store) {
+    constexpr int N = TX * TY;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    float acc[TY][TX];
+    bp2d_wave<KIND, 8, TX, TY>(X0, Y0, w, h, (unsigned)((size_t)na * wave / NW),
+                               (unsigned)((size_t)na * (wave + 1) / NW), na, nd, stride, sp, ang, acc, buf[wave]);
+#pragma unroll
+    for (int j = 0; j < TY; ++j)
+#pragma unroll
+        for (int i = 0; i < TX; ++i) buf[wave][(j * TX + i) * 64 + lane] = acc[j][i];
+    __syncthreads();
+    for (int p = wave; p < N; p += NW) {
+        float sum = buf[0][p * 64 + lane];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) sum += buf[k][p * 64 + lane];
+        const int X = X0 + (int)(lane & 7) + 8 * (p % TX), Y = Y0 + (int)(lane >> 3) + 8 * (p / TX);
+        if (X < (int)w && Y < (int)h) store(X, Y, sum);
     }
 }
 

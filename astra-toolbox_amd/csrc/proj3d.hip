@@ -1479,7 +1479,7 @@ bool bp3d_use_tiles(const Geom3D &g, int kernel, unsigned ss) {
     if (g.kind == ASTRA_AMD_GEOM_CYLCONE || bp3d_use_ss(g, kernel, ss) || !bp3d_zc(g, kernel)) return false;
     const char *e = std::getenv("ASTRA_AMD_BP3D_LDS");
     if (e && *e) return e[0] != '0';
-    return !std::getenv("ASTRA_AMD_BP3D_ZS") && bp3d_blocks(g) >= kBpFullBlocks;
+    return !std::getenv("ASTRA_AMD_BP3D_ZS") && (bp3d_blocks(g) >= kBpFullBlocks || bp3d_flat_ok(g));
 }
 
 // BP from the angle-major copy that bp3d_use_tiles names
@@ -1530,6 +1530,12 @@ void bp3d_run(const Geom3D &g, const float *copy, bool tiles, float *vol, float 
         const bool w2 = kernel == ASTRA_AMD_KER3D_2D_WEIGHTING;
         A.ang = (w2 ? g.bp_2d : g.bp_default).as<BP3DAngle>();
         A.aw = (w2 ? g.bp_w_2d : g.bp_w_default).as<float>();
+    }
+    if (tiles && bp3d_flat_ok(g) && !std::getenv("ASTRA_AMD_BP3D_LDS")) {
+        const bool w2 = kernel == ASTRA_AMD_KER3D_2D_WEIGHTING;
+        bp3d_flat_launch(g, A, (w2 ? g.bp_flat_2d : g.bp_flat_default).as<BP2DAngle>(), s);
+        prof_end(pt, s);
+        return;
     }
     const bool zc = bp3d_zc(g, kernel);
     const bool use_ss = bp3d_use_ss(g, kernel, ss);

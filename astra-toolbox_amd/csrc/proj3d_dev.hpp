@@ -254,6 +254,9 @@ void fp_group_launches(FPArgs A, unsigned tiles, unsigned count, K kern, hipStre
     }
 }
 
+// Flat parallel BP (bp3d_flat.hip)
+bool bp3d_flat_ok(const Geom3D &g);
+void bp3d_flat_launch(const Geom3D &g, const BPArgs &A, const BP2DAngle *ang, hipStream_t s);
 // Column FP (fp3d_cols.hip)
 size_t fp3d_cols_bytes(const Geom3D &g);
 void fp3d_cols_copy(const Geom3D &g, const float *vol, float *cols, hipStream_t s);
