@@ -306,12 +306,19 @@ int fp3d_cols_rays(const Geom3D &g, int grp) {
         return (64 * r - 1) * b.spread + (kSl - 1) * b.slope + 3.1 <= 64.0 * (r + 1);
     };
     if ((double)g.nu * g.nv / 64.0 * g.dir_count[grp] < 16384.0) return fits(2) ? 2 : fits(1) ? 1 : 0;
-    double best = per64[0] * ((g.nv + 15) / 16) / 4.0;
+    // Rays that do not climb keep their rows over all slices: the few rows past
+    // a window's last full block cost next to nothing, and the gather gains
+    // nothing from its smaller tiles (par3d, gather and columns: 400 x 397 x 130 / 300 x
+    // 513 x 140 4.5 and 3.3 ms, 256 x 253 x 100 / 120 x 300 x 100 0.80 and
+    // 0.58, 300 x 297 x 64 / 200 x 350 x 64 0.94 and 0.92, 300 x 297 x 290 /
+    // 200 x 350 x 200 with rows 1.5 apart 2.7 and 3.4).
+    double best = per64[0] * ((g.nv + 15) / 16) / 4.0 * (b.slope == 0.0 ? 1.25 : 1.0);
     int rays = 0;
     for (int r : {1, 2, 3, 4}) {
         if (!fits(r)) continue;
         // rows per ray beyond one cost their loads and interpolation
-        const double blocks = std::ceil(((64 * r - 1) * b.typical + 3.0) / 64.0) / r;
+        const double rows = ((64 * r - 1) * b.typical + 3.0) / 64.0;
+        const double blocks = (b.slope == 0.0 ? rows : std::ceil(rows)) / r;
         const double cost = (per64[r] + 0.5 * std::max(0.0, blocks - 1.0)) * r * ((g.nv + 64 * r - 1) / (64 * r));
         if (cost < best) {
             best = cost;
