@@ -477,6 +477,7 @@ struct Batch2D {
     bool weights_ready = false;
     double weights_relax = std::numeric_limits<double>::quiet_NaN();
     int fp_cfg = -1, bp_cfg = -1;
+    int fp_gather = 0;  // fastest of the gathering FP tilings
     // cached graph for (iterations, sinos, vols, lo, hi, fp_cfg, bp_cfg, stream)
     hipGraphExec_t exec = nullptr;
     int g_iters = -1;
@@ -740,6 +741,7 @@ void autotune(Batch2D &b, hipStream_t s) {
         if (ms < best_fp) {
             best_fp = ms;
             b.fp_cfg = k;
+            if (k < 3) b.fp_gather = k;
         }
     }
     float *vtmp = b.ones.as<float>();
@@ -782,9 +784,9 @@ void iterate(const Batch2D &b, const float *sinos, float *vols, int iters, float
 void build_persistent(Batch2D &b) {
     // the persistent kernel's tilings: the chosen ones, or for the
     // candidates it has no form of (LDS FP, pair and mixed FP, row-pair BP)
-    // the plain tiling of the same detectors / rows per thread (the same
-    // floats in every case)
-    static const int fp_plain[kFPCandidates] = {0, 1, 2, 0, 0, 1, 2};
+    // the plain tiling of the same detectors / rows per thread (LDS FP: the
+    // fastest plain one); the same floats in every case
+    const int fp_plain[kFPCandidates] = {0, 1, 2, b.fp_gather, 0, 1, 2};
     const int pf = fp_plain[b.fp_cfg], pb = b.bp_cfg < 6 ? b.bp_cfg : b.bp_cfg - 6;
     if (b.p_items.bytes() && b.p_fp == pf && b.p_bp == pb) return;
     const unsigned db = kFPDB[pf], py = kBPPY[pb % 3];
