@@ -104,11 +104,11 @@ struct AdjCols {
 };
 
 // grid = (slices / 4, row tiles, z tiles); 4 waves: 4 consecutive slices.
-// What bounds it: VALU issue (0.7 instructions per clock and CU, 39 per
-// (angle, u, slice) and 64 z) with LDS behind it (a read per candidate, 34 %).
-// 8 rows per wave: LDS lets 28 waves per CU run, 12 or 16 rows (17 and 16
-// waves) take 6.4 and 7.0 ms per 180 angles at 256^3 / 384^2, 8 rows 5.3, one
-// z per lane 8.7; the general gather takes 17.8.
+// What bounds it: VALU issue (0.7 instructions per clock and CU) with LDS
+// behind it (a read per candidate, 34 %).  8 rows per wave: LDS lets 28 waves
+// per CU run.  FP and gradient at 256^3 / 360 x 384^2 (two of these launches)
+// take 16.6 ms, 18.4 with 12 rows, 19.3 with 16, 22.9 with one z per lane, and
+// 42.4 with the general gather.
 template <int R>
 __global__ __launch_bounds__(256, 4) void adj_cols_kernel(AdjCols M) {
     __shared__ float acc_all[4][kRows][64 * R];

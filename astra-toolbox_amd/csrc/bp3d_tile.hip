@@ -169,7 +169,7 @@ __device__ __forceinline__ void bp_global_angle(const float *pl, unsigned pitch,
 // and LDS (two read2_b32, 80 % busy).  Measured at 512^3 / 720 x 768^2: 39 ms
 // against 48 for the gather.  Row pitch 72: neighbouring rows start 8 banks
 // apart (pitch 65: 54 ms, 64 and 96: 57 and 64, 76 and 80: 44 and 45).  48
-// rows hold 9 of 10 footprints there and leave LDS for 5 workgroups per CU
+// rows leave LDS for 5 workgroups per CU
 // (56 rows and 8 updates in flight, 4 workgroups: 44 ms; 40 rows, 6: 45 ms).
 template <int KIND, int ZS>
 __global__ __launch_bounds__(256, 5) void bp3d_tile_kernel(BPArgs A) {

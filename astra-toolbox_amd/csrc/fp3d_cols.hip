@@ -92,7 +92,7 @@ __device__ __forceinline__ int floor_i32(float x) {  // exact for |x| < 2^31
 // one of their two rows, so the waves of a workgroup are paced by a barrier
 // per chunk, and 4 waves per SIMD are faster than more.  Measured at 512^3 /
 // 720 x 768^2: 35 ms per group launch against 42 for the gather; without the
-// pacing 37 to 40, with 8 waves per workgroup 44, with 8 slices per chunk 36.
+// pacing 39, with 8 waves per workgroup 45, with 8 slices per chunk 37.
 template <int GK, int R>
 __global__ __launch_bounds__(64 * kWaves, 4) void fp3d_cols_kernel(FPArgs A, FPCols C) {
     constexpr int NB = R + 1;  // blocks of rows: R in flight, one more where a chunk needs it

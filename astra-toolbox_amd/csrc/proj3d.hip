@@ -727,7 +727,7 @@ __global__ __launch_bounds__(256) void bp3d_kernel(BPArgs A) {
 // wave adds their sums in the order of the waves.  A call's time here is one
 // wave's chain of angles (a load's latency each), so a quarter of the
 // angles, and four times the waves.  64^3 / 90 x 96^2: 96 us as 64 workgroups
-// of bp3d_kernel, 22 as 1024 of these.
+// of bp3d_kernel, 18 as 1024 of these.
 constexpr int kSplitZ = 4;
 template <int KIND, bool ZC>
 __global__ __launch_bounds__(256) void bp3d_split_kernel(BPArgs A) {
@@ -1234,7 +1234,9 @@ int bp_zs() {
 // 1070 ms per BP with 8 z voxels per thread (L2 hit rate 57 % at 40), 992
 // / 1001 ms for 40 / 80 with 16; at 512^3 / 720 x 768^2 (3.4 GB of padded
 // planes, 16 z voxels per thread), chunks of 90 / 180 / 240 / 360 / 720:
-// 49.5 / 48.6 / 48.2 / 48.7 / 49.3 ms.  So: 40 angles from 8 GiB
+// 49.5 / 48.6 / 48.2 / 48.7 / 49.3 ms with gathers of row pairs, chunks of
+// 180 / 240 / 360 / 720: 40.1 / 39.6 / 39.5 / 39.5 ms with staged tiles of the
+// plain planes (1.7 GB).  So: 40 angles from 8 GiB
 // of padded projections on; below that, equal chunks of at most 1.2 GB of
 // planes (a single launch below 1.2 GB); in every output mode.
 // ASTRA_AMD_BP3D_ACHUNK=<angles> forces a chunk size (0: default rule; read

@@ -655,18 +655,20 @@ def main():
         "texture_path": {
             "issued_lane_loads_per_launch": kd["issued_lane_loads_per_launch"],
             "issued_lane_loads_per_s": issued,
-            "limit_lane_loads_per_s": limits["taps"],
-            "coalesced_lane_loads_per_s": limits["coalesced"],
+            "limit_lane_loads_per_s": limits["coalesced"],
+            "gather_lane_loads_per_s": limits["taps"],
             "taps_2d_8byte_lane_loads_per_s": limits["taps_2d_8byte"],
             "tap_pairs_2d_16byte_align4_lane_loads_per_s": limits["tap_pairs_2d_16byte_align4"],
             "tap_pairs_2d_16byte_align8_lane_loads_per_s": limits["tap_pairs_2d_16byte_align8"],
             "ta_busy_frac": profile_value("ta_busy_frac", dom, n, na, nd),
-            "frac": issued / limits["taps"] if issued else None,
+            "frac": issued / limits["coalesced"] if issued else None,
+            "valu_issue_frac": profile_value("valu_issue_frac", dom, n, na, nd),
             "note": "issued = SQ_INSTS_VMEM_RD x 64 per launch (profile) over the live launch "
-                    "time; limit = astra_amd_calibrate_gather(mode 0) measured in this run: "
-                    "16-byte loads of a 16 x 4 ray bundle two thirds of a texel apart, from "
-                    "L1-resident data; ta_busy_frac = TA_BUSY_avr over the kernel's cycles "
-                    "(profile)"},
+                    "time; limit = astra_amd_calibrate_gather(mode 1) measured in this run: "
+                    "coalesced loads from L1-resident data, as the column FP and the staged BP "
+                    "issue them (gather_lane_loads_per_s: mode 0, one 16-byte load per tap); "
+                    "ta_busy_frac = TA_BUSY_avr over the kernel's cycles, valu_issue_frac = VALU "
+                    "wave-instructions per CU and cycle (profile)"},
     }
 
     fdk_s = None
