@@ -21,6 +21,20 @@ def test_same_storage_own_version(make):
     assert float(t.sum()) == 24.0 and not d.linked.requires_grad
 
 
+def _made_under_inference_mode():
+    with torch.inference_mode():
+        return torch.zeros(3, 4)
+
+
+def test_inference_tensor_is_written_outside_the_mode():
+    t = _made_under_inference_mode()
+    d = _link(t)
+    d.store(2.0)
+    d.write_back(torch.full((3, 4), 5.0))
+    assert d.linked.data_ptr() == t.data_ptr() and float(t.sum()) == 60.0
+    assert not d.linked.is_inference()
+
+
 @pytest.mark.parametrize("make", [
     lambda: torch.zeros(3, 4, requires_grad=True),
     lambda: torch.zeros(3, 4, dtype=torch.float64),
