@@ -405,11 +405,12 @@ def link_data(kind, geom, shape, obj):
     try:
         if type(obj) is torch.Tensor and obj.layout == torch.strided and not obj.requires_grad \
                 and obj.device.type in ("cpu", "cuda") \
-                and not (obj.is_conj() or obj.is_neg() or obj.is_inference()):
+                and not (obj.is_conj() or obj.is_neg() or obj.is_inference() or obj.is_nested or obj.has_names()):
             # what the exchange below gives for a plain tensor (the same
             # storage, a version counter of its own), without its 15 us; the
             # alias of an inference tensor is one too, which nothing outside
-            # that mode may write, the exchange's result a normal tensor
+            # that mode may write, the exchange's result a normal tensor;
+            # it drops names and refuses nested tensors, the alias does not
             t = obj.data
             t.data_ptr()  # a transform's wrapper has none: refused, as there
         else:

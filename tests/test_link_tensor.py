@@ -35,6 +35,15 @@ def test_inference_tensor_is_written_outside_the_mode():
     assert not d.linked.is_inference()
 
 
+@pytest.mark.filterwarnings("ignore:Named tensors")
+def test_named_tensor_links_without_its_names():
+    t = torch.zeros(3, 4, names=("row", "col"))
+    d = _link(t)
+    d.store(2.0)
+    assert d.linked.data_ptr() == t.data_ptr() and d.linked.names == (None, None)
+    assert float(t.rename(None).sum()) == 24.0
+
+
 @pytest.mark.parametrize("make", [
     lambda: torch.zeros(3, 4, requires_grad=True),
     lambda: torch.zeros(3, 4, dtype=torch.float64),
@@ -43,6 +52,7 @@ def test_inference_tensor_is_written_outside_the_mode():
     lambda: torch.zeros(3, 4, dtype=torch.complex64).conj().imag,
     lambda: torch.zeros(3, 4).to_sparse(),
     lambda: torch.zeros(3, 4, device="meta"),
+    lambda: torch.nested.nested_tensor([torch.zeros(4)] * 3),
 ])
 def test_refused(make):
     with pytest.raises(ValueError):
