@@ -552,7 +552,10 @@ __device__ __forceinline__ void fp2d_wave(int d0, int a0, unsigned na, unsigned 
 // extremes over the tile are at the corners, and the clamp is monotone),
 // widened by one texel on each side, far beyond the fp32 rounding of the
 // taps' incremental coordinates; 64 angles' intervals are computed at a
-// time, one per lane.  An angle whose interval exceeds kBp2Row texels, or
+// time, one per lane.  Corners are those of the tile's part inside the slice:
+// lanes past its right or bottom edge (nothing of theirs is stored) can
+// project anywhere, so a tile that the edge cuts clamps every tap to the
+// staged texels, as a tile that reaches the padded row's ends does.  An angle whose interval exceeds kBp2Row texels, or
 // whose denominator changes sign over the tile, is sampled from global memory.
 // Lanes in 8 x 8 squares: the footprint is short for the updates it serves,
 // and the taps of neighbouring lanes share LDS words.
@@ -567,10 +570,11 @@ constexpr int kBp2Row = 256;  // texels per staged angle row
 constexpr int kBp2Buf = kBp2KA * kBp2Row;  // floats per wave
 
 // Interval of an angle packed in an int: first texel | texels << 20 |
-// no tap is clamped << 30; texels 0: from global memory.
+// no tap is clamped << 30; texels 0: from global memory.  whole: the tile
+// lies inside the slice.
 template <int KIND>
 __device__ __forceinline__ int bp2d_footprint(const BP2DAngle &c, float fx0, float fx1, float fy0,
-                                              float fy1, float hi, int pitch) {
+                                              float fy1, float hi, int pitch, bool whole) {
     float tmin = INFINITY, tmax = -INFINITY, dmin = INFINITY, dmax = -INFINITY;
     for (int j = 0; j < 4; ++j) {
         const float fx = (j & 1) ? fx1 : fx0, fy = (j & 2) ? fy1 : fy0;
@@ -584,7 +588,7 @@ __device__ __forceinline__ int bp2d_footprint(const BP2DAngle &c, float fx0, flo
     }
     const bool sign_ok = KIND == 0 || KIND == 3 || dmin > 0.f || dmax < 0.f;
     if (!sign_ok || !__builtin_isfinite(tmin) || !__builtin_isfinite(tmax)) return 0;
-    const bool inner = tmin >= 1.5f && tmax <= hi - 1.f;
+    const bool inner = whole && tmin >= 1.5f && tmax <= hi - 1.f;
     // taps read texels floor(t) and floor(t) + 1 (t >= 0.5 after the clamp)
     const int t0 = max(0, (int)clamp_pad(tmin, hi) - 1);
     const int t1 = min(pitch - 1, (int)clamp_pad(tmax, hi) + 2);
@@ -593,9 +597,10 @@ __device__ __forceinline__ int bp2d_footprint(const BP2DAngle &c, float fx0, flo
 }
 
 // One angle's updates of a wave's tile; at: LDS byte address of texel 0 of
-// the angle's row (LDS), or the row's byte offset in rs.
+// the angle's row (LDS), or the row's byte offset in rs.  CLIP: tap
+// coordinates are clamped to [lo, hi].
 template <int KIND, int LX, int TX, int TY, bool CLIP, bool LDS>
-__device__ __forceinline__ void bp2d_angle(const BP2DAngle &c, float fx, float fy, float hi, unsigned at,
+__device__ __forceinline__ void bp2d_angle(const BP2DAngle &c, float fx, float fy, float lo, float hi, unsigned at,
                                            __amdgpu_buffer_rsrc_t rs, float (&acc)[TY][TX]) {
     typedef const __attribute__((address_space(3))) float *lptr;
     constexpr bool PAR = KIND == 0 || KIND == 3;
@@ -615,7 +620,7 @@ __device__ __forceinline__ void bp2d_angle(const BP2DAngle &c, float fx, float f
         for (int e = 0; e < G; ++e) {
             const float fr = PAR ? 1.f : __builtin_amdgcn_rcpf(den);
             float t = PAR ? num : num * fr;
-            if (CLIP) t = clamp_pad(t, hi);
+            if (CLIP) t = __builtin_amdgcn_fmed3f(t, lo, hi);  // (NaN: lo)
             if (LDS) {
                 const lptr q = (lptr)(size_t)(((unsigned)t << 2) + at);
                 q0[e] = q[0];
@@ -665,6 +670,7 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
     const float cx1 = min(X0 + LX * TX - 1, (int)w - 1) - 0.5f * w + 0.5f;
     const float cy0 = -(Y0 - 0.5f * h + 0.5f);
     const float cy1 = -(min(Y0 + 64 / LX * TY - 1, (int)h - 1) - 0.5f * h + 0.5f);
+    const bool whole = X0 + LX * TX <= (int)w && Y0 + 64 / LX * TY <= (int)h;
     const unsigned pitch = nd + 2 * kPad;
     const float hi = (float)nd + 2.5f;
     const unsigned step = (unsigned)stride * 4u;
@@ -687,7 +693,7 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
         const unsigned q = (a - alo) & 63;
         const __amdgpu_buffer_rsrc_t rs = rows(a);
         if (q == 0)
-            pk = bp2d_footprint<KIND>(ang[min(a + lane, na - 1)], cx0, cx1, cy0, cy1, hi, (int)pitch);
+            pk = bp2d_footprint<KIND>(ang[min(a + lane, na - 1)], cx0, cx1, cy0, cy1, hi, (int)pitch, whole);
 #pragma unroll
         for (int k = 0; k < kBp2KA; ++k) {
             in[k] = __builtin_amdgcn_readlane(pk, q + k);
@@ -729,11 +735,14 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
             c.w = cp[6];
             const unsigned at = __builtin_amdgcn_readfirstlane(lds + k * (kBp2Row * 4) - 4u * (f & 0xfffff));
             if (f >> 30)
-                bp2d_angle<KIND, LX, TX, TY, false, true>(c, fx, fy, hi, at, rs, acc);
-            else if (f >> 20)
-                bp2d_angle<KIND, LX, TX, TY, true, true>(c, fx, fy, hi, at, rs, acc);
-            else
-                bp2d_angle<KIND, LX, TX, TY, true, false>(c, fx, fy, hi, k * step, rs, acc);
+                bp2d_angle<KIND, LX, TX, TY, false, true>(c, fx, fy, 0.5f, hi, at, rs, acc);
+            else if (f >> 20) {
+                // texels [t0, t1]: a pixel of the slice has both its taps at
+                // least one texel inside, or is clamped to the row's ends, [0.5, hi]
+                const float t0 = (float)(f & 0xfffff), t1 = t0 + (float)((f >> 20) - 1);
+                bp2d_angle<KIND, LX, TX, TY, true, true>(c, fx, fy, t0 + 0.5f, t1 - 0.5f, at, rs, acc);
+            } else
+                bp2d_angle<KIND, LX, TX, TY, true, false>(c, fx, fy, 0.5f, hi, k * step, rs, acc);
         }
     }
 }

@@ -1,15 +1,21 @@
-"""The LDS-staged BPs take every tap from the rectangle they staged; that
-rectangle is the bounding box of the block's projected corners widened by
-one texel.  These CPU tests replay, in float32, the footprint arithmetic
-of `bp_footprint` (csrc/proj3d.hip) and `bp2d_footprint`
-(csrc/proj2d_dev.hpp) and the taps of the kernels (the same coefficient
-layout, fused multiply-adds and incremental z / row steps) over whole
-geometries, and check that every tap falls inside its staged rectangle --
-the property the kernels' index clamp relies on to never change a value.
-Planted mistakes (the footprint of the block's first z slice only, of the
-tile's first row only) must be caught.
+"""The staged BPs take every tap from the texels they staged, at LDS addresses
+that nothing checks: the footprint of a tile has to hold the taps of all its
+lanes, those past the edge of the volume included.
+
+These CPU tests compile the kernels' own text -- `bp_footprint` and
+`bp_tile_angle` of csrc/bp3d_tile.hip, `bp2d_footprint`, `bp2d_angle` and the
+lines of `bp2d_wave` that choose corners and clamps in csrc/proj2d_dev.hpp --
+for the host, with a checked pointer in the place of the LDS address, and
+run every lane of every tile over whole geometries.  Planted mistakes (the
+footprint of the block's first z slice, of the tile's first row; no clamp
+where a tile is cut by the slice's edge) must be caught.
 """
+import ctypes
 import math
+import os
+import re
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -17,129 +23,253 @@ import pytest
 from oracle import geometry as OG, proj3d as O3
 
 f32 = np.float32
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "astra-toolbox_amd", "csrc")
+
+PRELUDE = r"""
+#include <algorithm>
+#include <cmath>
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+using std::max;
+using std::min;
+#define __device__
+#define __forceinline__ inline
+constexpr int kPad = 2;
+typedef int __amdgpu_buffer_rsrc_t;
+struct float4 { float x, y, z, w; };
+static float4 make_float4(float x, float y, float z, float w) { return {x, y, z, w}; }
+struct BP2DAngle { float num[3], den[3], w, pad_; };
+struct BP3DAngle { float nu[4], nv[4], dn[4]; };
+static float med3(float x, float lo, float hi) {  // v_med3_f32: NaN gives the least of the others
+    return std::isnan(x) ? std::min(lo, hi) : std::min(std::max(x, lo), hi);
+}
+static float clamp_pad(float p, float hi) { return med3(p, 0.5f, hi); }
+static float frac(float p) { return p - std::floor(p); }
+static float lerp(float a, float b, float w) { return std::fma(w, b - a, a); }
+static float bilerp_pairs(float4 q, float w1, float w2) {
+    return lerp(std::fma(w2, q.y, q.x), std::fma(w2, q.w, q.z), w1);
+}
+static unsigned cvt_u32(float x) {  // v_cvt_u32_f32
+    return !(x > 0.f) ? 0u : x >= 4294967040.f ? 0xffffffffu : (unsigned)x;
+}
+static unsigned mul24(unsigned a, unsigned b) { return (a & 0xffffff) * (b & 0xffffff); }
+static float load_b32(int, int, int, int) { return 0.f; }
+// LDS pointer: counts the reads outside the staged texels [base, end)
+static unsigned lds_base, lds_end;
+static long outside;
+struct Lds {
+    unsigned a;
+    explicit Lds(size_t x) : a((unsigned)x) {}
+    float operator[](int i) const {
+        const unsigned p = a + 4u * (unsigned)i;
+        if (p < lds_base || p >= lds_end) ++outside;
+        return 0.f;
+    }
+};
+"""
+
+SUBST = [
+    (r"typedef const __attribute__\(\(address_space\(3\)\)\) float \*lptr;", "typedef Lds lptr;"),
+    (r"\(unsigned\)(t|pu|pv)\b", r"cvt_u32(\1)"),
+    (r"__builtin_amdgcn_fmed3f", "med3"),
+    (r"__builtin_amdgcn_rcpf\(", "(1.f / "),
+    (r"__builtin_amdgcn_raw_buffer_load_b32", "load_b32"),
+    (r"__int_as_float", ""),
+    (r"__umul24", "mul24"),
+    (r"__builtin_amdgcn_sched_barrier\(0\);", ""),
+    (r"__builtin_isfinite", "std::isfinite"),
+    (r'asm(?: volatile)?\("".*?\);', ""),
+]
 
 
-def fma(a, b, c):
-    """fp32 fused multiply-add (the product of two floats is exact in
-    float64; one rounding of the sum to float32)."""
-    return (np.asarray(a, np.float64) * np.asarray(b, np.float64) + np.asarray(c, np.float64)).astype(f32)
+def source(name):
+    return open(os.path.join(CSRC, name)).read()
 
 
-def clamp_pad(p, hi):
-    return np.minimum(np.maximum(p, f32(0.5)), f32(hi)).astype(f32)
+def part(text, first, last, include_last=False):
+    """`text` from the marker `first` to the marker `last`."""
+    a = text.index(first)
+    b = text.index(last, a) + (len(last) if include_last else 0)
+    return text[a:b]
+
+
+def host(text):
+    for pat, rep in SUBST:
+        text = re.sub(pat, rep, text, flags=re.S)
+    return text
+
+
+def harness_2d():
+    src = source("proj2d_dev.hpp")
+    code = part(src, "constexpr int kBp2KA", "// Sums over the angles [alo, ahi)")
+    corners = part(src, "    const float fx = (X0 + lane % LX)", "    const unsigned step")
+    call = re.search(r"pk = (bp2d_footprint<KIND>\(.*?\));\n", src).group(1)
+    call = re.sub(r"ang\[.*?\],", "c,", call, count=1)
+    choose = part(src, "            if (f >> 30)", "k * step, rs, acc);", True)
+    return host(code) + r"""
+template <int KIND, int LX, int TX, int TY>
+long run2d(unsigned w, unsigned h, unsigned na, unsigned nd, const BP2DAngle *ang, int plant, long *staged) {
+    outside = 0;
+    lds_base = 1u << 28;
+    for (int Y0 = 0; Y0 < (int)h; Y0 += 64 / LX * TY)
+        for (int X0 = 0; X0 < (int)w; X0 += LX * TX)
+            for (unsigned a = 0; a < na; ++a) {
+                const BP2DAngle c = ang[a];
+                for (int lane = 0; lane < 64; ++lane) {
+                    """ + host(corners).replace("const float cy1 =", "float cy1 =").replace(
+                        "const bool whole =", "bool whole =") + r"""
+                    if (plant == 1) cy1 = cy0;
+                    """ + ("if (plant == 2) whole = true;" if "bool whole" in corners else "") + r"""
+                    const int f = """ + call + r""";
+                    if (!(f >> 20)) break;
+                    if (lane == 0) ++*staged;
+                    lds_end = lds_base + 4u * ((f >> 20) & 0x3ff);
+                    const unsigned at = lds_base - 4u * (f & 0xfffff), k = 0, step = 0;
+                    const int rs = 0;
+                    float acc[TY][TX] = {};
+                    """ + host(choose) + r"""
+                }
+            }
+    return outside;
+}
+extern "C" long check2d(int kind, int form, unsigned w, unsigned h, unsigned na, unsigned nd, const BP2DAngle *ang,
+                        int plant, long *staged) {
+#define FORM(i, LX, TX, TY)                                                              \
+    if (form == i) return kind == 0 ? run2d<0, LX, TX, TY>(w, h, na, nd, ang, plant, staged) \
+                                    : run2d<1, LX, TX, TY>(w, h, na, nd, ang, plant, staged);
+    FORM(0, 8, 2, 2) FORM(1, 8, 4, 2) FORM(2, 8, 4, 4) FORM(3, 64, 1, 2) FORM(4, 64, 1, 4) FORM(5, 64, 1, 8)
+    return -1;
+}
+"""
+
+
+def harness_3d():
+    src = source("bp3d_tile.hip")
+    code = part(src, "constexpr int kTileRows", "}  // namespace") + \
+        part(src, "struct BPFoot {", "// Barrier that orders LDS only") + \
+        part(src, "template <int KIND, int ZS, bool CLIP>", "// The same from memory")
+    kernel = part(src, "void bp3d_tile_kernel(BPArgs A)", "// ---", False)
+    place = part(kernel, "    const unsigned tiles_x", "    const unsigned lds")
+    ray = part(kernel, "            const float un =", "            const float wgt")
+    zs = re.search(r"constexpr int kTileZ = (\d+);", source("proj3d_dev.hpp")).group(1)
+    return host(code) + "constexpr int ZS = " + zs + r""";
+struct Dim { unsigned x, y; };
+struct BPArgs { unsigned nx, ny, nz, nu, nv; };
+// one block of the launch at one angle; -1: not staged
+extern "C" long check3d(unsigned nx, unsigned ny, unsigned nz, unsigned nu, unsigned nv, const float *coef,
+                        unsigned bx, unsigned by, unsigned bz, int plant) {
+    constexpr int KIND = 0;
+    const BPArgs A{nx, ny, nz, nu, nv};
+    const Dim blockIdx{by * ((nx + 15) / 16) + bx, bz};
+    BP3DAngle c;
+    std::copy(coef, coef + 12, &c.nu[0]);
+    outside = 0;
+    lds_base = 1u << 28;
+    for (int wave = 0; wave < 4; ++wave)
+        for (int lane = 0; lane < 64; ++lane) {
+            """ + host(place).replace("const float cz0", "float cz0") + r"""
+            (void)active; (void)plane;
+            const BPFoot f = bp_footprint<KIND>(c, cx0, cx1, cy0, cy1, cz0, plant ? cz0 : cz1, hiu, hiv,
+                                                (int)pitch, (int)prow);
+            if (f.w == 0) return -1;
+            """ + host(ray) + r"""
+            // f.h rows of f.w staged texels, kTilePitch apart; a column outside its row can lie in
+            // another one: checked apart below
+            const unsigned at = lds_base + (unsigned)f.at;
+            lds_end = lds_base + 4u * ((f.h - 1) * kTilePitch + f.w);
+            float acc[ZS] = {};
+            f.inner ? bp_tile_angle<KIND, ZS, false>(c.nv[2], un, vn, fr, 1.f, hiu, hiv, at, acc)
+                    : bp_tile_angle<KIND, ZS, true>(c.nv[2], un, vn, fr, 1.f, hiu, hiv, at, acc);
+            const float pu = clamp_pad(un * fr, hiu);
+            if ((int)pu < f.u0 || (int)pu + 1 > f.u0 + f.w - 1) ++outside;
+        }
+    return outside;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("clang++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("footprints")
+    out = {}
+    for name, text in (("2d", harness_2d()), ("3d", harness_3d())):
+        cpp, so = d / (name + ".cpp"), d / (name + ".so")
+        cpp.write_text(PRELUDE + text)
+        r = subprocess.run([cxx, "-O2", "-std=c++17", "-mfma", "-ffp-contract=off", "-shared", "-fPIC", str(cpp),
+                            "-o", str(so)], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr
+        out[name] = ctypes.CDLL(str(so))
+        getattr(out[name], "check" + name).restype = ctypes.c_long
+    return out
 
 
 def bp3d_coeffs(vec, vs):
     """The kernel's float32 BP3DAngle (csrc/geometry.cpp cone_bp_coeffs):
     DevConeParams with the texel-centre offset and the padding folded in."""
     nu, nv, dn = O3.cone_bp_params(vec, "default", vs)
-    cu = np.array([nu[k] + 1.5 * dn[k] for k in range(4)], dtype=f32)
-    cv = np.array([nv[k] + 1.5 * dn[k] for k in range(4)], dtype=f32)
-    cd = np.array(dn, dtype=f32)
-    return cu, cv, cd
+    return np.array([[nu[k] + 1.5 * dn[k] for k in range(4)], [nv[k] + 1.5 * dn[k] for k in range(4)], dn],
+                    dtype=f32)
 
 
-def footprint3d(c, x0, x1, y0, y1, z0, z1, hiu, hiv, pitch, prow, margin=1):
-    cu, cv, cd = c
-    us, vs_, ds = [], [], []
-    for j in range(4):
-        x = x1 if j & 1 else x0
-        y = y1 if j & 2 else y0
-        un = fma(y, cu[1], fma(x, cu[0], cu[3]))
-        dn = fma(y, cd[1], fma(x, cd[0], cd[3]))
-        ds.append(dn)
-        fr = f32(1.0) / dn
-        us.append(clamp_pad(f32(un * fr), hiu))
-        for z in (z0, z1):
-            vn = fma(z, cv[2], fma(y, cv[1], fma(x, cv[0], cv[3])))
-            vs_.append(clamp_pad(f32(vn * fr), hiv))
-    if not (min(ds) > 0 or max(ds) < 0):
-        return None
-    u0 = max(0, int(min(us)) - margin)
-    u1 = min(pitch - 2, int(max(us)) + margin)
-    v0 = max(0, int(min(vs_)) - margin)
-    v1 = min(prow - 1, int(max(vs_)) + margin)
-    return u0, v0, u1 - u0 + 1, v1 - v0 + 1
-
-
-def check3d(n, na, nu, nv, sod, odd, blocks, zs=8, margin=1, angle_step=1, plant=False):
+def check3d(lib, shape, na, nu, nv, sod, odd, angle_step=1, plant=False):
+    nz, ny, nx = shape
     ang = np.linspace(0, 2 * np.pi, na, endpoint=False)
     vecs, vs = OG.normalise_3d(OG.gen_cone_projections(ang, nu, nv, sod, odd, 1.0, 1.0), "cone",
-                               OG.vol_geom_3d(n, n, n))
-    hiu, hiv = f32(nu + 2.5), f32(nv + 2.5)
-    pitch, prow = nu + 4, nv + 4
-    h = 0.5 * n - 0.5
-    bad = 0
+                               OG.vol_geom_3d(ny, nx, nz))
+    bad = staged = 0
+    pick = lambda n: sorted({0, n // 3, n // 2, n - 1})
     for a in range(0, na, angle_step):
         c = bp3d_coeffs(vecs[a], vs)
-        cu, cv, cd = c
-        for (bx, by, bz) in blocks:
-            X0, Y0, Z0 = bx * 16, by * 16, bz * zs
-            fp = footprint3d(c, f32(X0 - h), f32(min(X0 + 15, n - 1) - h), f32(Y0 - h),
-                             f32(min(Y0 + 15, n - 1) - h), f32(Z0 - h),
-                             f32(Z0 - h) if plant else f32(Z0 + zs - 1 - h),
-                             hiu, hiv, pitch, prow, margin)
-            if fp is None:
-                continue
-            u0, v0, w, hh = fp
-            X = np.arange(X0, min(X0 + 16, n))
-            Y = np.arange(Y0, min(Y0 + 16, n))
-            fx = (X.astype(f32) - f32(0.5 * n) + f32(0.5)).astype(f32)[None, :]
-            fy = (Y.astype(f32) - f32(0.5 * n) + f32(0.5)).astype(f32)[:, None]
-            fz = f32(f32(Z0) - f32(0.5 * n) + f32(0.5))
-            un = fma(fz, cu[2], fma(fy, cu[1], fma(fx, cu[0], cu[3])))
-            vn = fma(fz, cv[2], fma(fy, cv[1], fma(fx, cv[0], cv[3])))
-            dn = fma(fz, cd[2], fma(fy, cd[1], fma(fx, cd[0], cd[3])))
-            fr = (f32(1.0) / dn).astype(f32)
-            pu = clamp_pad((un * fr).astype(f32), hiu)
-            col = np.floor(pu).astype(int) - u0
-            bad += int(np.count_nonzero((col < 0) | (col > w - 1)))
-            for i in range(zs):
-                pv = clamp_pad((vn * fr).astype(f32), hiv)
-                row = np.floor(pv).astype(int) - v0
-                bad += int(np.count_nonzero((row < 0) | (row > hh - 1)))
-                vn = (vn + cv[2]).astype(f32)
+        p = c.ctypes.data_as(ctypes.c_void_p)
+        for bx in pick((nx + 15) // 16):
+            for by in pick((ny + 15) // 16):
+                for bz in pick((nz + 15) // 16):
+                    r = lib["3d"].check3d(nx, ny, nz, nu, nv, p, bx, by, bz, int(plant))
+                    staged += r >= 0
+                    bad += max(r, 0)
+    assert staged > 0
     return bad
 
 
-def _blocks(n, zs=8):
-    nb, nz = n // 16, n // zs
-    pick = sorted({0, nb // 3, nb // 2, nb - 1})
-    zpick = sorted({0, nz // 4, nz // 2, nz - 1})
-    return [(bx, by, bz) for bx in pick for by in pick for bz in zpick]
-
-
-def test_bp3d_taps_inside_staged_footprint_512():
+def test_bp3d_taps_inside_staged_footprint_512(lib):
     """The benchmarked cone geometry (512^3, 768^2, SOD 1000, ODD 500),
     corner / edge / centre blocks at every 6th of the 720 angles."""
-    assert check3d(512, 720, 768, 768, 1000.0, 500.0, _blocks(512), angle_step=6) == 0
+    assert check3d(lib, (512, 512, 512), 720, 768, 768, 1000.0, 500.0, angle_step=6) == 0
 
 
-def test_bp3d_taps_inside_staged_footprint_near_source():
-    assert check3d(48, 24, 96, 96, 40.0, 400.0, _blocks(48)) == 0
+def test_bp3d_taps_inside_staged_footprint_near_source(lib):
+    assert check3d(lib, (48, 48, 48), 24, 96, 96, 40.0, 400.0) == 0
 
 
-def test_bp3d_planted_first_slice_footprint_is_caught():
+def test_bp3d_taps_inside_staged_footprint_ragged(lib):
+    """Blocks cut by the volume's faces, a source near them."""
+    assert check3d(lib, (19, 47, 33), 60, 80, 72, 45.0, 60.0) == 0
+
+
+def test_bp3d_planted_first_slice_footprint_is_caught(lib):
     """A footprint from the block's first z slice only misses taps."""
-    assert check3d(64, 36, 96, 96, 150.0, 100.0, _blocks(64), plant=True) > 0
+    assert check3d(lib, (64, 64, 64), 36, 96, 96, 150.0, 100.0, plant=True) > 0
 
 
-def check2d(kind, w, h, nd, na, sod, odd, py, margin=1, wcap=256, plant=False):
+def bp2d_coeffs(kind, w, h, nd, na, sod, odd):
+    """The kernel's BP2DAngle (csrc/geometry.cpp angle2d_params), float32."""
     ang = np.linspace(0.2, 0.2 + 2 * np.pi, na, endpoint=False)
     vg = OG.vol_geom_2d(h, w)
     if kind == "par":
         vecs, _ = OG.normalise_2d(OG.gen_par_projections(ang, nd, 1.1), "parallel", vg)
     else:
         vecs, _ = OG.normalise_2d(OG.gen_fan_projections(ang, nd, sod, odd, 1.3), "fan", vg)
-    pitch, hi = nd + 4, f32(nd + 2.5)
-    bad = 0
+    out = np.zeros((na, 8), f32)
     for a in range(na):
         p = [float(x) for x in vecs[a]]
         if kind == "par":
             rx, ry, dsx, dsy, ux, uy = p
             d = ux * ry - uy * rx
-            num = np.array([(dsy * rx - dsx * ry) / d + 1.5, ry / d, -rx / d], dtype=f32)
-            den = np.array([1, 0, 0], dtype=f32)
+            out[a, :7] = [(dsy * rx - dsx * ry) / d + 1.5, ry / d, -rx / d, 1, 0, 0, 1]
         else:
             sx, sy, dsx, dsy, ux, uy = p
             smdx, smdy = sx - dsx, sy - dsy
@@ -147,65 +277,49 @@ def check2d(kind, w, h, nd, na, sod, odd, py, margin=1, wcap=256, plant=False):
             sc = math.sqrt(ux * ux + uy * uy) / det2(ux, uy, smdx, smdy)
             nc, nx, ny = sc * det2(sx, sy, dsx, dsy), sc * smdy, -sc * smdx
             dc, dx, dy = sc * det2(ux, uy, sx, sy), sc * uy, -sc * ux
-            num = np.array([nc + 1.5 * dc, nx + 1.5 * dx, ny + 1.5 * dy], dtype=f32)
-            den = np.array([dc, dx, dy], dtype=f32)
-        for X0 in range(0, w, 64):
-            for Yt0 in range(0, h, 4 * py):
-                cx = [f32(f32(X0) - f32(0.5 * w) + f32(0.5)),
-                      f32(f32(min(X0 + 63, w - 1)) - f32(0.5 * w) + f32(0.5))]
-                ylast = Yt0 if plant else min(Yt0 + 4 * py - 1, h - 1)
-                cy = [-f32(f32(Yt0) - f32(0.5 * h) + f32(0.5)),
-                      -f32(f32(ylast) - f32(0.5 * h) + f32(0.5))]
-                ts, ds = [], []
-                for j in range(4):
-                    fx, fy = cx[j & 1], cy[(j >> 1) & 1]
-                    nn = fma(fy, num[2], fma(fx, num[1], num[0]))
-                    dd = fma(fy, den[2], fma(fx, den[1], den[0]))
-                    ds.append(dd)
-                    fr = f32(1.0) if kind == "par" else f32(f32(1.0) / dd)
-                    ts.append(clamp_pad(f32(nn * fr), hi))
-                if kind != "par" and not (min(ds) > 0 or max(ds) < 0):
-                    continue
-                t0 = max(0, int(min(ts)) - margin)
-                t1 = min(pitch - 1, int(max(ts)) + 1 + margin)
-                if t1 - t0 + 1 > wcap:
-                    continue
-                X = np.arange(X0, min(X0 + 64, w))
-                fx = (X.astype(f32) - f32(0.5 * w) + f32(0.5)).astype(f32)
-                for Y0 in range(Yt0, min(Yt0 + 4 * py, h), py):
-                    fy0 = -f32(f32(Y0) - f32(0.5 * h) + f32(0.5))
-                    nn = fma(fy0, num[2], fma(fx, num[1], num[0]))
-                    dd = fma(fy0, den[2], fma(fx, den[1], den[0]))
-                    for i in range(py):
-                        if Y0 + i >= h:
-                            break
-                        fr = np.ones_like(dd) if kind == "par" else (f32(1.0) / dd).astype(f32)
-                        t = clamp_pad((nn * fr).astype(f32), hi)
-                        o = np.floor(t).astype(int) - t0
-                        bad += int(np.count_nonzero((o < 0) | (o > t1 - t0 - 1)))
-                        nn = (nn - num[2]).astype(f32)
-                        dd = (dd - den[2]).astype(f32)
+            out[a, :7] = [nc + 1.5 * dc, nx + 1.5 * dx, ny + 1.5 * dy, dc, dx, dy, 1]
+    return out
+
+
+# pixels of a tile: bp2d_tile_kernel's 16 x 16, 32 x 16, 32 x 32 and the
+# batched kernels' 64 columns of 2, 4, 8 rows
+FORMS = {"16x16": 0, "32x16": 1, "32x32": 2, "rows2": 3, "rows4": 4, "rows8": 5}
+
+
+def check2d(lib, kind, form, w, h, nd, na, sod, odd, plant=0):
+    c = bp2d_coeffs(kind, w, h, nd, na, sod, odd)
+    staged = ctypes.c_long(0)
+    bad = lib["2d"].check2d(0 if kind == "par" else 1, FORMS[form], w, h, na, nd,
+                            c.ctypes.data_as(ctypes.c_void_p), plant, ctypes.byref(staged))
+    assert bad >= 0 and staged.value > 0
     return bad
 
 
-@pytest.mark.parametrize("py", [2, 4, 8])
-@pytest.mark.parametrize("case", [("par", 130, 70, 200, 45, 0, 0), ("fan", 129, 97, 190, 60, 500.0, 300.0),
-                                  ("fan", 96, 96, 200, 50, 60.0, 400.0)],
-                         ids=["par", "fan", "fan_near"])
-def test_bp2d_taps_inside_staged_footprint(case, py):
-    kind, w, h, nd, na, sod, odd = case
-    assert check2d(kind, w, h, nd, na, sod, odd, py) == 0
+RAGGED = {"par": ("par", 130, 70, 200, 45, 0, 0), "fan": ("fan", 129, 97, 190, 60, 500.0, 300.0),
+          "fan_near": ("fan", 96, 96, 200, 50, 60.0, 400.0),
+          "par_cut": ("par", 65, 33, 40, 30, 0, 0), "fan_cut": ("fan", 70, 41, 64, 48, 44.0, 20.0)}
 
 
-def test_bp2d_planted_first_row_footprint_is_caught():
-    assert check2d("fan", 129, 97, 190, 60, 500.0, 300.0, 4, plant=True) > 0
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("case", RAGGED)
+def test_bp2d_taps_inside_staged_footprint(lib, case, form):
+    kind, w, h, nd, na, sod, odd = RAGGED[case]
+    assert check2d(lib, kind, form, w, h, nd, na, sod, odd) == 0
+
+
+def test_bp2d_planted_first_row_footprint_is_caught(lib):
+    assert check2d(lib, "fan", "32x32", 128, 96, 190, 60, 500.0, 300.0, plant=1) > 0
+
+
+def test_bp2d_planted_unclamped_cut_tile_is_caught(lib):
+    """Lanes past the slice of a tile that its edge cuts, without the clamp."""
+    assert check2d(lib, "par", "32x32", 130, 70, 200, 45, 0, 0, plant=2) > 0
 
 
 @pytest.mark.parametrize("case", [("par", 1024, 1024, 1536, 8, 0, 0), ("fan", 512, 512, 768, 12, 1024.0, 512.0)],
                          ids=["par1024", "fan512"])
-def test_bp2d_taps_inside_staged_footprint_batched_sizes(case):
+def test_bp2d_taps_inside_staged_footprint_batched_sizes(lib, case):
     """Slices of the batched workload's sizes (fan: source-origin 2N,
-    origin-detector N), 8 rows per thread: the staged taps read LDS without
-    a clamp, so every tap must stay inside its footprint."""
+    origin-detector N), 8 rows per thread."""
     kind, w, h, nd, na, sod, odd = case
-    assert check2d(kind, w, h, nd, na, sod, odd, 8) == 0
+    assert check2d(lib, kind, "rows8", w, h, nd, na, sod, odd) == 0
