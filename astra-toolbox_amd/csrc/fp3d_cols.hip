@@ -288,39 +288,85 @@ void fp3d_cols_copy(const Geom3D &g, const float *vol, float *cols, hipStream_t 
     AMX_LAUNCHED();
 }
 
+namespace {
+// Rows one chunk of group `grp` can need with r rays per lane: the rays'
+// spread, their drift over the chunk, and the two taps with the margins of
+// params().
+bool fits(const ColsBound &b, int r) {
+    return (64 * r - 1) * b.spread + (kSl - 1) * b.slope + 3.1 <= 64.0 * (r + 1);
+}
+double waves(const Geom3D &g, int grp, int r) {
+    return (double)g.nu * g.dir_count[grp] * ((g.nv + 64 * r - 1) / (64 * r));
+}
+// Rays per lane of a group whose launch does not fill the chip; 0: it does,
+// or columns do not serve it.
+int small_rays(const Geom3D &g, int grp) {
+    const ColsBound &b = g.cols[grp];
+    const int r = !b.ok || !g.dir_count[grp] ? 0 : g.nv > 64 && fits(b, 2) ? 2 : fits(b, 1) ? 1 : 0;
+    return r && waves(g, grp, r) < 16384.0 ? r : 0;
+}
+}  // namespace
+
 // Rays per lane of the column FP for direction group `grp`, 0: the gather.
-// The cost is the time per 64 rays of a column, relative to the gather with
-// its 16-row tiles, times the columns' blocks: measured at 512^3 / 768 rows
-// (43 ms per group launch for the gather; 43, 36, 35 with 2, 3, 4 rays per
-// lane; one ray per lane repeats the slice's work for each 64 rays) and at
-// 256^3 / 384 rows.  Below 16384 waves the chip is not full and a call is its
-// copies and one wave's slices: 2 rays per lane (64^3 / 90 x 96^2: FP and BP
-// 319 us, 1 ray per lane 335, gather 385 with its two copies).
+//
+// A column wave holds 64 R rows whatever the detector has, so the waves to
+// count are nu x angles x blocks of 64 R rows.  From 16384 of them on the chip is
+// full and the cost is the time per 64 rows of a column, relative to the
+// gather with its 16-row tiles, times the columns' blocks: measured at 512^3 /
+// 768 rows (43 ms per group launch for the gather; 43, 36, 35 with 2, 3, 4 rays
+// per lane; one ray per lane repeats the slice's work for each 64 rows) and at
+// 256^3 / 384 rows.
+//
+// Below, a launch is its copies, a chain of n slices per wave and what its
+// waves add to that: the time of an FP in us, fitted to 320 shapes (n x n x nz
+// with n 32 to 512, 6 to 360 angles, 1 to 128 rows, cone and parallel).  The
+// gather's waves are 4 x 16 rays and end at once where none is on the
+// detector; its pair copies cost 0.6 us per 10^6 voxels and group more.  The
+// groups that do not fill the chip are decided together: one in each form
+// pays for the copies of both.  Gather and columns: 64^2 x 6 / 90 x 83 x 8
+// 73 and 49, 256^2 x 12 / 90 x 332 x 16 164 and 382, 512^2 x 12 / 24 x 665 x
+// 16 208 and 538, x 48 / 24 x 665 x 64 673 and 551, 64^2 x 72 / 90 x 83 x 96
+// 120 and 59.  Over 688 shapes, 288 of them not in the fit, the form taken is
+// at most 1.09 times slower than the gather (geometric mean 0.74).
 int fp3d_cols_rays(const Geom3D &g, int grp) {
     const ColsBound &b = g.cols[grp];
     if (!b.ok) return 0;
+    if (const int r0 = small_rays(g, grp)) {
+        const double rows = g.nv > 12 ? 4.0 * ((g.nv + 15) / 16) : (g.nv + 3) / 4;
+        double cols = 0.0, gather = 0.0;
+        for (int k = 0; k < 2; ++k) {
+            const int r = small_rays(g, k);
+            if (!r) continue;
+            const double n = 0.5 * (k == 0 ? g.nx : g.ny);
+            const bool level = g.cols[k].slope == 0.0;
+            const double chain = level ? 0.34 : 0.32, each = (level ? 65e-6 : 85e-6) * (r == 2 ? 1.2 : 1.0);
+            cols += 7.5 + n * (chain + each * waves(g, k, r));
+            gather += 26.5 + n * (0.25 + 98e-6 * ((g.nu + 15) / 16) * rows * g.dir_count[k]) +
+                      0.6e-6 * g.nx * g.ny * g.nz;
+        }
+        return cols < 0.96 * gather ? r0 : 0;
+    }
+    const bool level = b.slope == 0.0;  // rays that do not climb
     const double per64[5] = {1.0, 1.2, 1.0, 0.84, 0.82};
-    auto fits = [&](int r) {
-        // rows one chunk can need: the rays' spread, their drift over the
-        // chunk, and the two taps with the margins of params()
-        return (64 * r - 1) * b.spread + (kSl - 1) * b.slope + 3.1 <= 64.0 * (r + 1);
-    };
-    if ((double)g.nu * g.nv / 64.0 * g.dir_count[grp] < 16384.0) return fits(2) ? 2 : fits(1) ? 1 : 0;
     // Rays that do not climb keep their rows over all slices: the few rows past
     // a window's last full block cost next to nothing, and the gather gains
     // nothing from its smaller tiles (par3d, gather and columns: 400 x 397 x 130 / 300 x
     // 513 x 140 4.5 and 3.3 ms, 256 x 253 x 100 / 120 x 300 x 100 0.80 and
     // 0.58, 300 x 297 x 64 / 200 x 350 x 64 0.94 and 0.92, 300 x 297 x 290 /
-    // 200 x 350 x 200 with rows 1.5 apart 2.7 and 3.4).
-    double best = per64[0] * ((g.nv + 15) / 16) / 4.0 * (b.slope == 0.0 ? 1.25 : 1.0);
+    // 200 x 350 x 200 with rows 1.5 apart 2.7 and 3.4).  With one ray per lane
+    // that holds up to about 32768 waves: 512^2 x 48 / 90 x 665 x 64 (29925) 1.49
+    // and 1.27, 256^2 x 48 / 360 x 332 x 64 (59760) 0.98 and 1.15 ms.
+    const double base = per64[0] * ((g.nv + 15) / 16) / 4.0;
+    double best = INFINITY;
     int rays = 0;
     for (int r : {1, 2, 3, 4}) {
-        if (!fits(r)) continue;
+        if (!fits(b, r)) continue;
         // rows per ray beyond one cost their loads and interpolation
         const double rows = ((64 * r - 1) * b.typical + 3.0) / 64.0;
-        const double blocks = (b.slope == 0.0 ? rows : std::ceil(rows)) / r;
+        const double blocks = (level ? rows : std::ceil(rows)) / r;
         const double cost = (per64[r] + 0.5 * std::max(0.0, blocks - 1.0)) * r * ((g.nv + 64 * r - 1) / (64 * r));
-        if (cost < best) {
+        const double limit = level && (r > 1 || waves(g, grp, r) < 32768.0) ? 1.25 * base : base;
+        if (cost < std::min(best, limit)) {
             best = cost;
             rays = r;
         }
