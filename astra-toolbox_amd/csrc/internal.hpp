@@ -180,6 +180,9 @@ struct Geom3D {
     // detector), so the BP hoists them out of its z loop
     bool zc_default = false, zc_fdk = false, zc_2d = false;
     ColsBound cols[3];
+    // zc_default: share of the BP's blocks and angles whose detector footprint
+    // does not fit the staged tile (bp3d_tile_miss)
+    float tile_miss = 1.f;
     // par3d with horizontal rays and a vertical detector, the same rows at
     // every angle: the BP is a 2D BP of each detector row and an
     // interpolation at row flat_v[0] * z + flat_v[1] (z from the centre,
@@ -307,6 +310,8 @@ void xpby_ratio_launch(float *p, const float *z, size_t n, const double *num, co
                        hipStream_t s);
 
 // geometry helpers
+float bp3d_tile_miss(int kind, unsigned nx, unsigned ny, unsigned nz, unsigned nu, unsigned nv,
+                     const BP3DAngle *ang, unsigned na);
 Geom3D *geom3d_build(int kind, unsigned nx, unsigned ny, unsigned nz, unsigned na, unsigned nu,
                      unsigned nv, const double *vecs, const float *vol_scale);
 Geom2D *geom2d_build(int kind, unsigned w, unsigned h, unsigned na, unsigned nd,

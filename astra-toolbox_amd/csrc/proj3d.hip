@@ -1481,7 +1481,7 @@ bool bp3d_use_tiles(const Geom3D &g, int kernel, unsigned ss) {
     if (g.kind == ASTRA_AMD_GEOM_CYLCONE || bp3d_use_ss(g, kernel, ss) || !bp3d_zc(g, kernel)) return false;
     const char *e = std::getenv("ASTRA_AMD_BP3D_LDS");
     if (e && *e) return e[0] != '0';
-    return !std::getenv("ASTRA_AMD_BP3D_ZS") && (bp3d_blocks(g) >= kBpFullBlocks || bp3d_flat_ok(g));
+    return !std::getenv("ASTRA_AMD_BP3D_ZS") && ((bp3d_blocks(g) >= kBpFullBlocks && bp3d_tiles_fit(g)) || bp3d_flat_ok(g));
 }
 
 // BP from the angle-major copy that bp3d_use_tiles names

@@ -274,5 +274,6 @@ void adj3d_cols_add(const Geom3D &g, const float *cols, float *vol, hipStream_t 
 // bp3d_kernel's, kTileZ voxels of a column per thread.
 constexpr int kTileZ = 16;
 void bp3d_tile_launch(int kind, const BPArgs &A, hipStream_t s);
+bool bp3d_tiles_fit(const Geom3D &g);
 
 }  // namespace amx

@@ -58,10 +58,10 @@ def test_tile_bp_equals_gather(case, monkeypatch):
     y = torch.rand((nv, na, nu), generator=g, device="cuda")
     pid = astra.create_projector("cuda3d", pg, vg)
     out = {}
-    for lds in ("0", None):
+    for lds in ("0", "1", None):  # gather, tiles, the one the rule takes
         monkeypatch.setenv("ASTRA_AMD_BP3D_LDS", lds) if lds else monkeypatch.delenv("ASTRA_AMD_BP3D_LDS")
         out[lds] = torch.full((nz, ny, nx), float("nan"), dtype=torch.float32, device="cuda")
         astra.experimental.direct_BP3D(pid, out[lds], y)
     astra.projector3d.delete(pid)
     assert float(out["0"].abs().max()) > 0
-    assert torch.equal(out["0"], out[None])
+    assert torch.equal(out["0"], out["1"]) and torch.equal(out["0"], out[None])

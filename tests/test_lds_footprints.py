@@ -34,6 +34,7 @@ PRELUDE = r"""
 using std::max;
 using std::min;
 #define __device__
+#define __host__
 #define __forceinline__ inline
 constexpr int kPad = 2;
 typedef int __amdgpu_buffer_rsrc_t;
