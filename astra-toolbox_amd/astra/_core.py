@@ -403,9 +403,9 @@ def link_data(kind, geom, shape, obj):
     if isinstance(obj, np.ndarray) and not obj.flags.writeable:
         raise ValueError("Failed to link dlpack array: read-only arrays are not supported")
     try:
-        if type(obj) is torch.Tensor and obj.layout == torch.strided and not obj.requires_grad \
-                and obj.device.type in ("cpu", "cuda") \
-                and not (obj.is_conj() or obj.is_neg() or obj.is_inference() or obj.is_nested or obj.has_names()):
+        if type(obj) is torch.Tensor and obj.dtype is torch.float32 and obj.layout is torch.strided \
+                and (obj.is_cuda or obj.is_cpu) and not (obj.requires_grad or obj.is_neg() or obj.is_inference()
+                                                         or obj.is_nested or obj.has_names()):
             # what the exchange below gives for a plain tensor (the same
             # storage, a version counter of its own), without its 15 us; the
             # alias of an inference tensor is one too, which nothing outside
