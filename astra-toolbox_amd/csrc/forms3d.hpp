@@ -1,0 +1,25 @@
+// Host rules that choose the 3D kernels' forms from a geometry (host code
+// only: no device code or launch).
+#pragma once
+
+#include "internal.hpp"
+
+namespace amx {
+
+// Column FP (fp3d_cols.hip): rays per lane for a direction group, 0: the gather
+int fp3d_cols_rays(const Geom3D &g, int grp);
+
+struct FPForms {
+    int rays[3] = {0, 0, 0};  // per direction group, as fp3d_cols_rays
+    bool cols = false, gather = false;
+    size_t bytes = 0;  // the volume copies' scratch
+};
+FPForms fp3d_forms(const Geom3D &g, unsigned ss);
+
+// Whether the BP's detector footprints fit the staged tiles (bp3d_tile.hip)
+bool bp3d_tiles_fit(const Geom3D &g);
+
+// Flat parallel BP (bp3d_flat.hip)
+bool bp3d_flat_ok(const Geom3D &g);
+
+}  // namespace amx

@@ -1322,6 +1322,24 @@ FPArgs fp_args(const Geom3D &g, int grp, float out_scale) {
 
 }  // namespace
 
+// The forms of a call's direction groups.  Groups whose detector columns run
+// along z take the column FP (ASTRA_AMD_FP3D_LDS, when set, picks one of the
+// gather's two forms).  One buffer holds every group's copy of the volume in
+// turn, so a call's scratch is its largest copy.  The columns' is half the
+// z-group's row pairs: the largest row-pair copy of any group, which
+// composite.py plans with, bounds it.
+FPForms fp3d_forms(const Geom3D &g, unsigned ss) {
+    FPForms f;
+    const bool cols_on = ss == 1 && g.kind != ASTRA_AMD_GEOM_CYLCONE && !std::getenv("ASTRA_AMD_FP3D_LDS");
+    for (int k = 0; k < 3; ++k) {
+        if (!g.dir_count[k]) continue;
+        f.rays[k] = cols_on ? fp3d_cols_rays(g, k) : 0;
+        (f.rays[k] ? f.cols : f.gather) = true;
+        f.bytes = std::max(f.bytes, f.rays[k] ? fp3d_cols_bytes(g) : group_elems(g, k) * sizeof(float2));
+    }
+    return f;
+}
+
 void fp3d_launch(const Geom3D &g, const float *vol, float *proj, float out_scale, int mode,
                  const float *resid_b, const float *resid_w, bool padded_out, hipStream_t s,
                  unsigned ss) {
@@ -1329,39 +1347,22 @@ void fp3d_launch(const Geom3D &g, const float *vol, float *proj, float out_scale
     // the cylindrical-detector FP has no sub-rays (ConeCylFP ignores
     // iRaysPerDetDim, cuda/3d/cone_cyl.cu:613-666)
     if (g.kind == ASTRA_AMD_GEOM_CYLCONE) ss = 1;
-    // groups whose detector columns run along z take the column FP
-    // (ASTRA_AMD_FP3D_LDS, when set, picks one of the gather's two forms)
-    const bool cols_on = ss == 1 && !std::getenv("ASTRA_AMD_FP3D_LDS");
-    size_t need = 0;
-    int groups[3], ng = 0, rays[3] = {0, 0, 0};
-    bool cols = false;
-    for (int k = 0; k < 3; ++k)
-        if (g.dir_count[k]) {
-            rays[k] = cols_on ? fp3d_cols_rays(g, k) : 0;
-            if (rays[k])
-                cols = true;
-            else
-                need = std::max(need, group_elems(g, k) * sizeof(float2));
-            groups[ng++] = k;
-        }
-    std::unique_ptr<Scratch> colv, copy, tick;
-    if (cols) {
-        colv.reset(new Scratch(fp3d_cols_bytes(g), s));
-        fp3d_cols_copy(g, vol, colv->as<float>(), s);
-    }
-    if (need) {
-        copy.reset(new Scratch(need, s));                  // row-pair copy
-        tick.reset(new Scratch(8 * kTickPitch * sizeof(unsigned), s));  // ticket counters of the resident FP grid
-    }
-    for (int i = 0; i < ng; ++i) {
-        const int k = groups[i];
-        if (!rays[k]) make_group_copy(g, k, vol, copy->as<float2>(), s);
+    const FPForms f = fp3d_forms(g, ss);
+    Scratch copy(f.bytes, s);
+    std::unique_ptr<Scratch> tick;  // ticket counters of the resident FP grid
+    if (f.gather) tick.reset(new Scratch(8 * kTickPitch * sizeof(unsigned), s));
+    if (f.cols) fp3d_cols_copy(g, vol, copy.as<float>(), s);
+    // the column groups first: the row-pair copies then overwrite theirs
+    for (int i = 0; i < 6; ++i) {
+        const int k = i % 3;
+        if (!g.dir_count[k] || (f.rays[k] != 0) != (i < 3)) continue;
+        if (!f.rays[k]) make_group_copy(g, k, vol, copy.as<float2>(), s);
         FPArgs A = fp_args(g, k, out_scale);
         // march3d's buffer loads address a slice at 32-bit scalar offsets
         // of up to 3 slices
         AMX_REQUIRE((size_t)(A.n1 + 2 * kPad) * (A.n2 + 2 * kPad) * sizeof(float2) <= (1ull << 30),
                     "fp3d: volume slice too large (%u x %u)", A.n1, A.n2);
-        A.volp = rays[k] ? nullptr : copy->as<float>();
+        A.volp = f.rays[k] ? nullptr : copy.as<float>();
         A.out = proj;
         A.rb = resid_b;
         A.rw = resid_w;
@@ -1374,8 +1375,8 @@ void fp3d_launch(const Geom3D &g, const float *vol, float *proj, float out_scale
                                                                      : "fp3d_par3d",
                                   (double)g.dir_count[k] * g.nu * g.nv * A.n0 * ss * ss, s);
         A.ss = ss;
-        if (rays[k]) {
-            fp3d_cols_launch(g, k, rays[k], A, colv->as<float>(), s);
+        if (f.rays[k]) {
+            fp3d_cols_launch(g, k, f.rays[k], A, copy.as<float>(), s);
             prof_end(pt, s);
             continue;
         }

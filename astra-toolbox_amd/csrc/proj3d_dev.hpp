@@ -9,6 +9,7 @@
 #include <cstdlib>
 
 #include "devutil.hpp"
+#include "forms3d.hpp"
 #include "internal.hpp"
 
 namespace amx {
@@ -255,12 +256,10 @@ void fp_group_launches(FPArgs A, unsigned tiles, unsigned count, K kern, hipStre
 }
 
 // Flat parallel BP (bp3d_flat.hip)
-bool bp3d_flat_ok(const Geom3D &g);
 void bp3d_flat_launch(const Geom3D &g, const BPArgs &A, const BP2DAngle *ang, hipStream_t s);
 // Column FP (fp3d_cols.hip)
 size_t fp3d_cols_bytes(const Geom3D &g);
 void fp3d_cols_copy(const Geom3D &g, const float *vol, float *cols, hipStream_t s);
-int fp3d_cols_rays(const Geom3D &g, int grp);
 void fp3d_cols_launch(const Geom3D &g, int grp, int rays, FPArgs A, const float *cols, hipStream_t s);
 
 // Its transpose (adj3d_cols.hip)
@@ -274,6 +273,5 @@ void adj3d_cols_add(const Geom3D &g, const float *cols, float *vol, hipStream_t 
 // bp3d_kernel's, kTileZ voxels of a column per thread.
 constexpr int kTileZ = 16;
 void bp3d_tile_launch(int kind, const BPArgs &A, hipStream_t s);
-bool bp3d_tiles_fit(const Geom3D &g);
 
 }  // namespace amx

@@ -16,10 +16,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 DRIVER = r"""
 #include "internal.hpp"
-namespace amx {
-int fp3d_cols_rays(const Geom3D &g, int grp);
-bool bp3d_tiles_fit(const Geom3D &g);
-}
+#include "forms3d.hpp"
 using namespace amx;
 static void fill(Geom3D &g, const unsigned *n) {
     g.kind = ASTRA_AMD_GEOM_CONE;
@@ -38,6 +35,19 @@ extern "C" int cols_rays(const unsigned *n, double spread, double typical, doubl
         g.cols[k].slope = slope;
     }
     return fp3d_cols_rays(g, 0);
+}
+// bytes of the FP's volume copies; ok: the groups that columns can serve
+extern "C" size_t fp_scratch(const unsigned *n, int ok, int *rays) {
+    Geom3D g;
+    fill(g, n);
+    g.dir_count[0] = g.dir_count[1] = (int)n[3] / 2;
+    for (int k = 0; k < 2; ++k) {
+        g.cols[k].ok = (ok >> k) & 1;
+        g.cols[k].spread = g.cols[k].typical = 1.0;
+    }
+    const FPForms f = fp3d_forms(g, 1);
+    for (int k = 0; k < 3; ++k) rays[k] = f.rays[k];
+    return f.bytes;
 }
 // ang: na rows of BP3DAngle
 extern "C" int tiles_fit(const unsigned *n, const BP3DAngle *ang, double *miss) {
@@ -65,7 +75,9 @@ def rules(tmp_path_factory):
                         _lib.LIB_PATH, "-Wl,-rpath," + os.path.dirname(_lib.LIB_PATH)],
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
-    return ctypes.CDLL(so)
+    lib = ctypes.CDLL(so)
+    lib.fp_scratch.restype = ctypes.c_size_t
+    return lib
 
 
 def cols_rays(rules, shape, level=False):
@@ -128,3 +140,15 @@ def test_bp_tiles_only_where_footprints_fit(rules, n, na, nu, du, sod, odd, shar
     got = rules.tiles_fit((ctypes.c_uint * 6)(n, n, n, na, nu, nu), c.ctypes.data_as(ctypes.c_void_p),
                           ctypes.byref(miss))
     assert abs(miss.value - share) <= 0.07 and bool(got) == fits
+
+
+@pytest.mark.parametrize("ok", [0, 1, 2, 3])
+@pytest.mark.parametrize("shape", [(600, 200, 400, 720, 900, 500), (64, 48, 50, 90, 96, 96), (3, 700, 300, 200, 900, 400),
+                                   (1, 1, 500, 100, 5, 700)])
+def test_fp_scratch_is_what_the_planner_counts(rules, shape, ok):
+    """Groups of different forms use one buffer in turn."""
+    from astra import composite
+    rays = (ctypes.c_int * 3)()
+    got = rules.fp_scratch((ctypes.c_uint * 6)(*shape), ok, rays)
+    assert all(not r or (ok >> k) & 1 for k, r in enumerate(rays))
+    assert 0 < got <= composite._fp_scratch(shape[2::-1])

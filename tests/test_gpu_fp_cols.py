@@ -61,6 +61,30 @@ def test_cols_fp_helical():
     _check(pg, vg, OG.conevec_from_astra(rows, nu, nv), "cone", (nx, ny, nz), nu, nv)
 
 
+def test_groups_of_both_forms_share_one_buffer():
+    """Upright detectors in the x-group, tilted ones in the y-group: the
+    columns' and the gather's copies of the volume use one buffer in turn, no
+    more scratch than the job splitter counts."""
+    import astra
+    import torch
+    from astra import _lib, composite
+    from oracle import geometry as OG
+    nx, ny, nz, nu, nv = 44, 40, 72, 50, 65
+    vg = astra.create_vol_geom(ny, nx, nz)
+    rows = []
+    for a in np.linspace(0.1, 0.1 + 2 * np.pi, 60, endpoint=False):
+        c, s = np.cos(a), np.sin(a)
+        t = 0.0 if abs(s) > abs(c) else 0.1
+        rows.append([130 * s, -130 * c, 0, -60 * s, 60 * c, 0, c, s, 0, -t * s, t * c, 1.0])
+    rows = np.array(rows)
+    pg = astra.create_proj_geom("cone_vec", nv, nu, rows)
+    torch.cuda.synchronize()
+    base, _ = _lib.scratch_usage(reset_peak=True)
+    _check(pg, vg, OG.conevec_from_astra(rows, nu, nv), "cone", (nx, ny, nz), nu, nv)
+    _, peak = _lib.scratch_usage()
+    assert peak - base <= composite._fp_scratch((nz, ny, nx)) + 65536  # tickets, allocation grain
+
+
 def _check(pg, vg, vec, kind, n, nu, nv):
     import astra
     import torch
