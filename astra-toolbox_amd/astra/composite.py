@@ -62,6 +62,23 @@ def _bp_scratch(pshape):
     return na * (nv + 2 * _PAD) * (nu + 2 * _PAD) * 8
 
 
+def _matched_tables(pshape, ss):
+    """Bytes of the matched BP's ray tables per angle and at most: those of
+    its general or its split form, whichever is larger, for the angles of a
+    pass (128 MiB of tables, or one angle)."""
+    nv, na, nu = pshape
+    nv, nu = nv * ss, nu * ss
+    split = nu * (nv * 4 + 24)
+    per = max(nu * nv * 20, split)
+    n = max(1, min(na, (128 << 20) // split, 32768))
+    return per + 48, min(per * n, max(128 << 20, per)) + 48 * n
+
+
+def _matched_scratch(vshape, pshape, ss=1):
+    """Bytes of the matched BP's ray tables and its split form's sums."""
+    return _matched_tables(pshape, ss)[1] + _nbytes(vshape)
+
+
 def _nbytes(shape):
     return int(np.prod(shape)) * 4
 
@@ -94,24 +111,33 @@ def plan_fp(vshape, pshape, cap, vol_on_host=True, proj_on_host=True):
     return plan
 
 
-def plan_bp(vshape, pshape, cap, vol_on_host=True, proj_on_host=True):
-    """[(z range, [angle ranges])] of a split BP, or None when it fits."""
-    need = _bp_scratch(pshape) + (_nbytes(vshape) if vol_on_host else 0) + \
+def plan_bp(vshape, pshape, cap, vol_on_host=True, proj_on_host=True, matched_ss=0):
+    """[(z range, [angle ranges])] of a split BP, or None when it fits.
+    matched_ss: rays per detector pixel and dimension of a matched BP (0:
+    another kernel)."""
+    scratch = _matched_scratch(vshape, pshape, matched_ss) if matched_ss else _bp_scratch(pshape)
+    need = scratch + (_nbytes(vshape) if vol_on_host else 0) + \
         (_nbytes(pshape) if proj_on_host else 0)
     if need <= cap:
         return None
     nv, na, nu = pshape
     nz, ny, nx = vshape
-    per_slice = nx * ny * 4
+    # a slab and, of a matched BP, its sums
+    per_slice = nx * ny * 4 * (2 if matched_ss else 1)
     out_cap = cap // 3 if proj_on_host else cap // 2
     slabs = _chunks(nz, out_cap // per_slice)
-    per_angle = (nv + 2 * _PAD) * (nu + 2 * _PAD) * 8 + (nv * nu * 4 if proj_on_host else 0)
+    part = nv * nu * 4 if proj_on_host else 0
+    per_angle = (nv + 2 * _PAD) * (nu + 2 * _PAD) * 8 + part
     plan = []
     for z0, z1 in slabs:
-        rest = cap - (z1 - z0) * per_slice
-        if rest < per_angle:
+        if cap - (z1 - z0) * nx * ny * 4 < per_angle:
             raise AstraError("BP job does not fit in %d bytes of GPU memory" % cap)
-        plan.append(((z0, z1), _chunks(na, rest // per_angle)))
+        rest = cap - (z1 - z0) * per_slice
+        per = rest // per_angle
+        if matched_ss:  # tables that grow with the angles, or full ones
+            one, full = _matched_tables(pshape, matched_ss)
+            per = max(rest // (one + part), (rest - full) // part if part else (na if rest >= full else 0))
+        plan.append(((z0, z1), _chunks(na, per)))
     return plan
 
 
@@ -274,8 +300,9 @@ def bp(p, dproj, dvol, mode, kernel=None):
     vol_host, proj_host = _host_array(dvol), _host_array(dproj)
     plan = None
     if vol_host is not None or proj_host is not None:
+        matched = (p.kernel if kernel is None else kernel) == _lib.KER3D_MATCHED_BP
         plan = plan_bp(p.vol_shape, p.proj_shape, budget(dev), vol_host is not None,
-                       proj_host is not None)
+                       proj_host is not None, p.detector_ss if matched else 0)
     if plan is None:
         s = dproj.on_device(dev)
         v = dvol.on_device(dev, init=(mode == MODE_ADD))

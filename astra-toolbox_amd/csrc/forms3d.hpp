@@ -16,6 +16,17 @@ struct FPForms {
 };
 FPForms fp3d_forms(const Geom3D &g, unsigned ss);
 
+// Its transpose (adj3d_cols.hip)
+bool adj3d_cols_ok(const Geom3D &g, int grp);
+
+// The matched BP's forms and scratch bytes
+struct MatchedForms {
+    bool cols[3] = {false, false, false};  // per direction group: split, else gather
+    unsigned chunk[3] = {0, 0, 0};         // angles per pass
+    size_t tables = 0, geo = 0, sums = 0;
+};
+MatchedForms matched_forms(const Geom3D &g, unsigned ss);
+
 // Whether the BP's detector footprints fit the staged tiles (bp3d_tile.hip)
 bool bp3d_tiles_fit(const Geom3D &g);
 

@@ -1630,6 +1630,30 @@ static int matched_slices() {
     return v;
 }
 
+// Groups whose detector columns run along z split into a pass over u and one
+// over v (ASTRA_AMD_MATCHED_SLICES, when set, asks for the general gather);
+// their sums are kept z-fastest, one volume more, and added to it at the end.
+// Ray tables are built per chunk of angles, at most 128 MiB at a time (one
+// angle at least): they are scratch of every gradient step of the
+// differentiable projector.  composite.py plans with an upper bound of both.
+MatchedForms matched_forms(const Geom3D &g, unsigned ss) {
+    MatchedForms f;
+    const size_t NU = (size_t)g.nu * ss, NV = (size_t)g.nv * ss;
+    const bool cols_on = ss == 1 && g.kind != ASTRA_AMD_GEOM_CYLCONE && !std::getenv("ASTRA_AMD_MATCHED_SLICES");
+    for (int k = 0; k < 3; ++k) {
+        if (!g.dir_count[k]) continue;
+        f.cols[k] = cols_on && adj3d_cols_ok(g, k);
+        const size_t per = f.cols[k] ? NU * (NV * sizeof(float) + sizeof(float4) + sizeof(float2))
+                                     : NU * NV * (sizeof(float4) + sizeof(float));
+        const size_t n = std::min<size_t>(g.na, (size_t(128) << 20) / per);
+        f.chunk[k] = (unsigned)std::max<size_t>(1, std::min<size_t>(n, 32768));
+        f.tables = std::max(f.tables, per * f.chunk[k]);
+        f.geo = std::max(f.geo, f.chunk[k] * 3 * sizeof(float4));
+        if (f.cols[k]) f.sums = (size_t)g.nx * g.ny * g.nz * sizeof(float);
+    }
+    return f;
+}
+
 void bp3d_matched_launch(const Geom3D &g, const float *proj, float *vol, float out_scale,
                          int mode, hipStream_t s, unsigned ss) {
     AMX_REQUIRE(ss >= 1 && ss <= 16, "bp3d: rays per detector dimension must be in [1, 16]");
@@ -1641,48 +1665,20 @@ void bp3d_matched_launch(const Geom3D &g, const float *proj, float *vol, float o
     // 32-bit byte offsets into one angle's ray table
     AMX_REQUIRE(NU * NV * sizeof(float4) < (1ull << 32),
                 "bp3d: detector too large for the matched adjoint");
-    // ray tables are built per chunk of angles, at most 128 MiB at a time
-    // (one angle at least): the tables are scratch of every gradient step
-    // of the differentiable projector, so they stay small beside the data
-    const size_t per_angle = NU * NV * (sizeof(float4) + sizeof(float));
-    const size_t per_angle_cols = NU * (NV * sizeof(float) + sizeof(float4) + sizeof(float2));
-    auto chunk_of = [&](size_t per) {
-        const size_t n = std::min<size_t>(g.na, (size_t(128) << 20) / per);
-        return (unsigned)std::max<size_t>(1, std::min<size_t>(n, 32768));
-    };
+    const MatchedForms f = matched_forms(g, ss);
     const bool cyl = g.kind == ASTRA_AMD_GEOM_CYLCONE;
-    // groups whose detector columns run along z split into a pass over u and
-    // one over v (ASTRA_AMD_MATCHED_SLICES, when set, asks for the general
-    // gather); their sums are kept z-fastest and added to vol at the end
-    const bool cols_on = ss == 1 && !cyl && !std::getenv("ASTRA_AMD_MATCHED_SLICES");
-    bool cols[3], any_cols = false, any_gather = false;
-    for (int k = 0; k < 3; ++k) {
-        cols[k] = cols_on && g.dir_count[k] && adj3d_cols_ok(g, k);
-        any_cols |= cols[k];
-        any_gather |= g.dir_count[k] && !cols[k];
-    }
-    size_t bytes = 0;
-    unsigned most = 1;
-    if (any_gather) {
-        bytes = per_angle * chunk_of(per_angle);
-        most = chunk_of(per_angle);
-    }
-    if (any_cols) {
-        bytes = std::max(bytes, per_angle_cols * chunk_of(per_angle_cols));
-        most = std::max(most, chunk_of(per_angle_cols));
-    }
-    Scratch rays(bytes, s), geo((size_t)most * 3 * sizeof(float4), s);
+    Scratch rays(f.tables, s), geo(f.geo, s);
     std::unique_ptr<Scratch> colv;
-    if (any_cols) {
-        colv.reset(new Scratch(nvox * sizeof(float), s));
+    if (f.sums) {
+        colv.reset(new Scratch(f.sums, s));
         fill_launch(colv->as<float>(), nvox, 0.f, s);
     }
     for (int k = 0; k < 3; ++k) {
         if (!g.dir_count[k]) continue;
-        const unsigned chunk = chunk_of(cols[k] ? per_angle_cols : per_angle);
+        const unsigned chunk = f.chunk[k];
         FPArgs A = fp_args(g, k, out_scale);
         A.ss = ss;
-        if (cols[k]) {
+        if (f.cols[k]) {
             float4 *q0 = rays.as<float4>();
             float2 *q1 = reinterpret_cast<float2 *>(q0 + NU * chunk);
             float *yw = reinterpret_cast<float *>(q1 + NU * chunk);
@@ -1750,7 +1746,7 @@ void bp3d_matched_launch(const Geom3D &g, const float *proj, float *vol, float o
             AMX_LAUNCHED();
         }
     }
-    if (any_cols) adj3d_cols_add(g, colv->as<float>(), vol, s);
+    if (f.sums) adj3d_cols_add(g, colv->as<float>(), vol, s);
 }
 
 }  // namespace amx

@@ -263,7 +263,6 @@ void fp3d_cols_copy(const Geom3D &g, const float *vol, float *cols, hipStream_t 
 void fp3d_cols_launch(const Geom3D &g, int grp, int rays, FPArgs A, const float *cols, hipStream_t s);
 
 // Its transpose (adj3d_cols.hip)
-bool adj3d_cols_ok(const Geom3D &g, int grp);
 void adj3d_cols_launch(const Geom3D &g, int grp, const FPArgs &A, const float *proj, const float4 *geo,
                        float4 *q0, float2 *q1, float *yw, float *out, hipStream_t s);
 void adj3d_cols_add(const Geom3D &g, const float *cols, float *vol, hipStream_t s);

@@ -42,6 +42,31 @@ def test_fp_bp_plans_tile_and_fit(seed):
     assert C.plan_fp(vshape, pshape, 10 ** 13) is None and C.plan_bp(vshape, pshape, 10 ** 13) is None
 
 
+@pytest.mark.parametrize("ss", [1, 2])
+@pytest.mark.parametrize("on_host", [True, False])
+@pytest.mark.parametrize("seed", range(6))
+def test_matched_bp_plans_fit(seed, on_host, ss):
+    """A matched BP's parts hold their ray tables and one more slab."""
+    rng = np.random.default_rng(seed)
+    vshape = tuple(int(x) for x in rng.integers(8, 300, 3))
+    pshape = tuple(int(x) for x in rng.integers(8, 400, 3))
+    nv, na, nu = pshape
+    nz, ny, nx = vshape
+    proj = C._nbytes(pshape) if on_host else 0
+    full = C._matched_scratch(vshape, pshape, ss) + C._nbytes(vshape) + proj
+    assert C.plan_bp(vshape, pshape, full, True, on_host, ss) is None
+    cap = int(full * rng.uniform(0.4, 0.95))
+    plan = C.plan_bp(vshape, pshape, cap, True, on_host, ss)
+    slabs = [r for r, _ in plan]
+    assert slabs[0][0] == 0 and slabs[-1][1] == nz and all(a[1] == b[0] for a, b in zip(slabs, slabs[1:]))
+    for (z0, z1), chunks in plan:
+        assert chunks[0][0] == 0 and chunks[-1][1] == na
+        for a0, a1 in chunks:
+            slab, part = (z1 - z0, ny, nx), (nv, a1 - a0, nu)
+            use = C._nbytes(slab) + (C._nbytes(part) if on_host else 0) + C._matched_scratch(slab, part, ss)
+            assert use <= cap
+
+
 def test_sub_geometries():
     vg = astra.create_vol_geom(8, 9, 10, -5, 4, -3, 5, -2.5, 7.5)
     parts = [C.vol_slab_geom(vg, z0, z1) for z0, z1 in ((0, 3), (3, 7), (7, 10))]

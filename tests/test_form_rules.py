@@ -49,6 +49,18 @@ extern "C" size_t fp_scratch(const unsigned *n, int ok, int *rays) {
     for (int k = 0; k < 3; ++k) rays[k] = f.rays[k];
     return f.bytes;
 }
+extern "C" size_t matched_scratch(const unsigned *n, int kind, int ok, unsigned ss) {
+    Geom3D g;
+    fill(g, n);
+    g.kind = kind;
+    g.dir_count[0] = g.dir_count[1] = (int)n[3] / 2;
+    for (int k = 0; k < 2; ++k) {
+        g.cols[k].ok = (ok >> k) & 1;
+        g.cols[k].spread = g.cols[k].typical = g.cols[k].closest = 1.0;
+    }
+    const MatchedForms f = matched_forms(g, ss);
+    return f.tables + f.geo + f.sums;
+}
 // ang: na rows of BP3DAngle
 extern "C" int tiles_fit(const unsigned *n, const BP3DAngle *ang, double *miss) {
     Geom3D g;
@@ -76,7 +88,7 @@ def rules(tmp_path_factory):
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
     lib = ctypes.CDLL(so)
-    lib.fp_scratch.restype = ctypes.c_size_t
+    lib.fp_scratch.restype = lib.matched_scratch.restype = ctypes.c_size_t
     return lib
 
 
@@ -152,3 +164,17 @@ def test_fp_scratch_is_what_the_planner_counts(rules, shape, ok):
     got = rules.fp_scratch((ctypes.c_uint * 6)(*shape), ok, rays)
     assert all(not r or (ok >> k) & 1 for k, r in enumerate(rays))
     assert 0 < got <= composite._fp_scratch(shape[2::-1])
+
+
+@pytest.mark.parametrize("ss", [1, 3])
+@pytest.mark.parametrize("ok", [0, 1, 3])
+@pytest.mark.parametrize("shape", [(256, 256, 256, 360, 384, 384), (600, 200, 400, 720, 900, 500),
+                                   (400, 400, 300, 4, 128, 100), (64, 48, 50, 90, 96, 96), (64, 48, 50, 90, 96, 1),
+                                   (20, 20, 20, 2, 3000, 3000)])
+def test_matched_scratch_is_what_the_planner_counts(rules, shape, ok, ss):
+    from astra import _lib, composite
+    nx, ny, nz, na, nu, nv = shape
+    for kind in (_lib.GEOM_CONE, _lib.GEOM_PAR3D):
+        got = rules.matched_scratch((ctypes.c_uint * 6)(*shape), kind, ok, ss)
+        assert 0 < got <= composite._matched_scratch((nz, ny, nx), (nv, na, nu), ss)
+    assert got >= (nx * ny * nz * 4 if ok and ss == 1 else 0)
