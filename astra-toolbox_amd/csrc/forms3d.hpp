@@ -27,6 +27,13 @@ struct MatchedForms {
 };
 MatchedForms matched_forms(const Geom3D &g, unsigned ss);
 
+// Workgroups of the BP's 16 x 16 column kernels with 16 z voxels per thread.
+// Below 1024 (4 per CU) the chip is not full: bp3d_split_kernel.
+inline size_t bp3d_blocks(const Geom3D &g) {
+    return (size_t)((g.nx + 15) / 16) * ((g.ny + 15) / 16) * ((g.nz + 15) / 16);
+}
+constexpr size_t kBpFullBlocks = 1024;
+
 // Whether the BP's detector footprints fit the staged tiles (bp3d_tile.hip)
 bool bp3d_tiles_fit(const Geom3D &g);
 

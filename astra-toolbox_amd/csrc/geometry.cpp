@@ -12,6 +12,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "forms3d.hpp"
 #include "internal.hpp"
 
 namespace amx {
@@ -390,7 +391,7 @@ Geom3D *geom3d_build(int kind, unsigned nx, unsigned ny, unsigned nz, unsigned n
     g->zc_fdk = !cyl && zconst(bf);
     g->zc_2d = !cyl && zconst(b2);
     for (int k = 0; k < 3; ++k) g->cols[k] = cols_bound(*g, k);
-    if (g->zc_default)
+    if (g->zc_default && bp3d_blocks(*g) >= kBpFullBlocks)
         g->tile_miss = bp3d_tile_miss(kind == ASTRA_AMD_GEOM_CONE ? 0 : 2, nx, ny, nz, nu, nv, bd.data(), na);
     // (a difference below the rounding of a row's coordinate is none)
     g->flat = kind == ASTRA_AMD_GEOM_PAR3D && g->zc_default && g->zc_2d;

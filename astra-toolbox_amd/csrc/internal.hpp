@@ -180,8 +180,9 @@ struct Geom3D {
     // detector), so the BP hoists them out of its z loop
     bool zc_default = false, zc_fdk = false, zc_2d = false;
     ColsBound cols[3];
-    // zc_default: share of the BP's blocks and angles whose detector footprint
-    // does not fit the staged tile (bp3d_tile_miss)
+    // zc_default and a volume that fills the chip: share of the BP's blocks and
+    // angles whose detector footprint does not fit the staged tile
+    // (bp3d_tile_miss, 50 us)
     float tile_miss = 1.f;
     // par3d with horizontal rays and a vertical detector, the same rows at
     // every angle: the BP is a 2D BP of each detector row and an

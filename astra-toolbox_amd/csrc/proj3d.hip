@@ -1446,12 +1446,13 @@ void bp3d_dispatch(int kind, bool zc, const BPArgs &A, hipStream_t s) {
         zc ? bp3d_kernel<2, ZS, true><<<grid, 256, 0, s>>>(A) : bp3d_kernel<2, ZS, false><<<grid, 256, 0, s>>>(A);
 }
 
-// Supersampling applies
-// to the default cone kernel and to par3d, as in ConeBP_Array / Par3DBP_Array
-// (cuda/3d/cone_bp.cu:351-370, cuda/3d/par3d_bp.cu:285-293).
+// Supersampling applies to the default cone kernel and to par3d, as in
+// ConeBP_Array / Par3DBP_Array (cuda/3d/cone_bp.cu:351-370,
+// cuda/3d/par3d_bp.cu:285-293).
 bool bp3d_use_ss(const Geom3D &g, int kernel, unsigned ss) {
     return ss > 1 && (g.kind != ASTRA_AMD_GEOM_CONE || kernel == ASTRA_AMD_KER3D_DEFAULT);
 }
+
 void bp3d_split_dispatch(int kind, bool zc, const BPArgs &A, hipStream_t s) {
     const dim3 grid(((A.nx + 7) / 8) * ((A.ny + 7) / 8), (A.nz + kSplitZ - 1) / kSplitZ);
     if (kind == 0)
@@ -1468,21 +1469,18 @@ bool bp3d_zc(const Geom3D &g, int kernel) {
     if (g.kind == ASTRA_AMD_GEOM_CONE && kernel == ASTRA_AMD_KER3D_FDK_WEIGHTING) return g.zc_fdk;
     return kernel == ASTRA_AMD_KER3D_2D_WEIGHTING ? g.zc_2d : g.zc_default;
 }
+
 // Whether a BP runs on the padded single layout of the projections with
-// footprints staged in LDS (bp3d_tile.hip); the others read their row-pair
-// copy.  ASTRA_AMD_BP3D_LDS=0 asks for the gather, 1 for the staged form (read
-// at every launch), ASTRA_AMD_BP3D_ZS, a property of the gather, for the gather.
-// Workgroups of the 16 x 16 column kernels with 16 z voxels per thread.  Below
-// 1024 (4 per CU) the chip is not full: bp3d_split_kernel.
-size_t bp3d_blocks(const Geom3D &g) {
-    return (size_t)((g.nx + 15) / 16) * ((g.ny + 15) / 16) * ((g.nz + 15) / 16);
-}
-constexpr size_t kBpFullBlocks = 1024;
+// footprints staged in LDS (bp3d_tile.hip) or as 2D BPs of the detector rows
+// (bp3d_flat.hip); the others read their row-pair copy.  ASTRA_AMD_BP3D_LDS=0
+// asks for the gather, 1 for the staged form (read at every launch),
+// ASTRA_AMD_BP3D_ZS, a property of the gather, for the gather.
 bool bp3d_use_tiles(const Geom3D &g, int kernel, unsigned ss) {
     if (g.kind == ASTRA_AMD_GEOM_CYLCONE || bp3d_use_ss(g, kernel, ss) || !bp3d_zc(g, kernel)) return false;
     const char *e = std::getenv("ASTRA_AMD_BP3D_LDS");
     if (e && *e) return e[0] != '0';
-    return !std::getenv("ASTRA_AMD_BP3D_ZS") && ((bp3d_blocks(g) >= kBpFullBlocks && bp3d_tiles_fit(g)) || bp3d_flat_ok(g));
+    if (std::getenv("ASTRA_AMD_BP3D_ZS")) return false;
+    return (bp3d_blocks(g) >= kBpFullBlocks && bp3d_tiles_fit(g)) || bp3d_flat_ok(g);
 }
 
 // BP from the angle-major copy that bp3d_use_tiles names
