@@ -641,8 +641,9 @@ __global__ __launch_bounds__(256) void fp3d_sumsq_kernel(FPArgs A) {
 }
 
 // ------------------------------------------------------------- BP --------
+// A column of ZS voxels from (X, Y, Z0): the sums over the angles a0, a0 + step,
+// ... of the launch, every tap gathered from the row-pair copy.
 // KIND: 0 cone fr^2 (default / FDK), 1 cone fr (2D weighting), 2 par3d.
-// One thread per (x, y) column of ZS voxels; 16 x 16 threads per group.
 // The angle loop is uniform, so the per-angle coefficients are scalar loads
 // and the angle's projection plane base is a scalar address.
 // ZC: U and the denominator are constant along z for every angle (checked
@@ -650,7 +651,6 @@ __global__ __launch_bounds__(256) void fp3d_sumsq_kernel(FPArgs A) {
 // tap offset and weight and the voxel weight are then computed once per
 // column and angle.  Both forms take the same fp32 operations on the same
 // values (adding a zero increment is exact), so they give identical results.
-// Sums over the angles a0, a0 + step, ... of the launch.
 template <int KIND, int ZS, bool ZC>
 __device__ __forceinline__ void bp_gather_column(const BPArgs &A, int X, int Y, int Z0, unsigned a0, unsigned step,
                                                  float (&acc)[ZS]) {
@@ -710,6 +710,7 @@ __device__ __forceinline__ void bp_gather_column(const BPArgs &A, int X, int Y, 
     }
 }
 
+// One thread per column; 16 x 16 threads per group.
 template <int KIND, int ZS, bool ZC>
 __global__ __launch_bounds__(256) void bp3d_kernel(BPArgs A) {
     const unsigned tiles_x = (A.nx + 15) / 16;
