@@ -552,10 +552,11 @@ __device__ __forceinline__ void fp2d_wave(int d0, int a0, unsigned na, unsigned 
 // extremes over the tile are at the corners, and the clamp is monotone),
 // widened by one texel on each side, far beyond the fp32 rounding of the
 // taps' incremental coordinates; 64 angles' intervals are computed at a
-// time, one per lane.  Corners are those of the tile's part inside the slice:
-// lanes past its right or bottom edge (nothing of theirs is stored) can
-// project anywhere, so a tile that the edge cuts clamps every tap to the
-// staged texels, as a tile that reaches the padded row's ends does.  An angle whose interval exceeds kBp2Row texels, or
+// time, one per lane.  The corners are the whole tile's, also where the slice's
+// edge cuts it: the lanes past the edge store nothing, but read their taps
+// from LDS like the others.  If the interval of one of the 64 angles cannot
+// be staged (a source just outside the slice), the corners are those of the
+// part inside, and every tap is clamped to the staged texels.  An angle whose interval exceeds kBp2Row texels, or
 // whose denominator changes sign over the tile, is sampled from global memory.
 // Lanes in 8 x 8 squares: the footprint is short for the updates it serves,
 // and the taps of neighbouring lanes share LDS words.
@@ -570,8 +571,8 @@ constexpr int kBp2Row = 256;  // texels per staged angle row
 constexpr int kBp2Buf = kBp2KA * kBp2Row;  // floats per wave
 
 // Interval of an angle packed in an int: first texel | texels << 20 |
-// no tap is clamped << 30; texels 0: from global memory.  whole: the tile
-// lies inside the slice.
+// no tap is clamped << 30; texels 0: from global memory.  whole: all of the
+// tile's lanes lie within the corners.
 template <int KIND>
 __device__ __forceinline__ int bp2d_footprint(const BP2DAngle &c, float fx0, float fx1, float fy0,
                                               float fy1, float hi, int pitch, bool whole) {
@@ -665,14 +666,19 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
     const unsigned lds = (unsigned)(size_t)(__attribute__((address_space(3))) float *)buf;
     const float fx = (X0 + lane % LX) - 0.5f * w + 0.5f;
     const float fy = -((Y0 + lane / LX) - 0.5f * h + 0.5f);  // world y
-    // corner pixels of the tile inside the slice
-    const float cx0 = X0 - 0.5f * w + 0.5f;
-    const float cx1 = min(X0 + LX * TX - 1, (int)w - 1) - 0.5f * w + 0.5f;
-    const float cy0 = -(Y0 - 0.5f * h + 0.5f);
-    const float cy1 = -(min(Y0 + 64 / LX * TY - 1, (int)h - 1) - 0.5f * h + 0.5f);
-    const bool whole = X0 + LX * TX <= (int)w && Y0 + 64 / LX * TY <= (int)h;
     const unsigned pitch = nd + 2 * kPad;
     const float hi = (float)nd + 2.5f;
+    auto interval = [&](const BP2DAngle &c) {
+        const float cx0 = X0 - 0.5f * w + 0.5f, cy0 = -(Y0 - 0.5f * h + 0.5f);
+        int f = 0, X1 = X0 + LX * TX - 1, Y1 = Y0 + 64 / LX * TY - 1;
+#pragma unroll 1
+        for (bool all = true;; all = false) {
+            f = bp2d_footprint<KIND>(c, cx0, X1 - 0.5f * w + 0.5f, cy0, -(Y1 - 0.5f * h + 0.5f), hi, (int)pitch, all);
+            if (!all || __all(f != 0) || (X1 < (int)w && Y1 < (int)h)) return f;
+            X1 = min(X1, (int)w - 1);
+            Y1 = min(Y1, (int)h - 1);
+        }
+    };
     const unsigned step = (unsigned)stride * 4u;
     // rows a .. a + kBp2KA - 1, as far as they exist
     auto rows = [&](unsigned a) {
@@ -693,7 +699,7 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
         const unsigned q = (a - alo) & 63;
         const __amdgpu_buffer_rsrc_t rs = rows(a);
         if (q == 0)
-            pk = bp2d_footprint<KIND>(ang[min(a + lane, na - 1)], cx0, cx1, cy0, cy1, hi, (int)pitch, whole);
+            pk = interval(ang[min(a + lane, na - 1)]);
 #pragma unroll
         for (int k = 0; k < kBp2KA; ++k) {
             in[k] = __builtin_amdgcn_readlane(pk, q + k);
@@ -737,7 +743,7 @@ __device__ __forceinline__ void bp2d_wave(int X0, int Y0, unsigned w, unsigned h
             if (f >> 30)
                 bp2d_angle<KIND, LX, TX, TY, false, true>(c, fx, fy, 0.5f, hi, at, rs, acc);
             else if (f >> 20) {
-                // texels [t0, t1]: a pixel of the slice has both its taps at
+                // texels [t0, t1]: a pixel within the corners has both its taps at
                 // least one texel inside, or is clamped to the row's ends, [0.5, hi]
                 const float t0 = (float)(f & 0xfffff), t1 = t0 + (float)((f >> 20) - 1);
                 bp2d_angle<KIND, LX, TX, TY, true, true>(c, fx, fy, t0 + 0.5f, t1 - 0.5f, at, rs, acc);

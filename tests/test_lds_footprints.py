@@ -7,8 +7,8 @@ These CPU tests compile the kernels' own text -- `bp_footprint` and
 lines of `bp2d_wave` that choose corners and clamps in csrc/proj2d_dev.hpp --
 for the host, with a checked pointer in the place of the LDS address, and
 run every lane of every tile over whole geometries.  Planted mistakes (the
-footprint of the block's first z slice, of the tile's first row; no clamp
-where a tile is cut by the slice's edge) must be caught.
+footprint of the block's first z slice, of the tile's first row, of the part
+of a tile inside the slice) must be caught.
 """
 import ctypes
 import math
@@ -56,6 +56,9 @@ static unsigned cvt_u32(float x) {  // v_cvt_u32_f32
 }
 static unsigned mul24(unsigned a, unsigned b) { return (a & 0xffffff) * (b & 0xffffff); }
 static float load_b32(int, int, int, int) { return 0.f; }
+// a vote of a wave's lanes, each with an angle of its own
+static bool others_fit = true;
+static bool __all(bool x) { return x && others_fit; }
 // LDS pointer: counts the reads outside the staged texels [base, end)
 static unsigned lds_base, lds_end;
 static long outside;
@@ -105,23 +108,26 @@ def harness_2d():
     src = source("proj2d_dev.hpp")
     code = part(src, "constexpr int kBp2KA", "// Sums over the angles [alo, ahi)")
     corners = part(src, "    const float fx = (X0 + lane % LX)", "    const unsigned step")
-    call = re.search(r"pk = (bp2d_footprint<KIND>\(.*?\));\n", src).group(1)
-    call = re.sub(r"ang\[.*?\],", "c,", call, count=1)
+    call = re.search(r"pk = (\w+\()ang\[.*?\]\);\n", src).group(1) + "c)"
     choose = part(src, "            if (f >> 30)", "k * step, rs, acc);", True)
+    whole = "Y1 = Y0 + 64 / LX * TY - 1;"  # the corners of the first try
+    assert corners.count(whole) == 1
+    corners = corners.replace(whole, whole + """
+        if (plant == 1) Y1 = Y0;
+        if (plant == 2) X1 = min(X1, (int)w - 1), Y1 = min(Y1, (int)h - 1);
+""")
     return host(code) + r"""
 template <int KIND, int LX, int TX, int TY>
 long run2d(unsigned w, unsigned h, unsigned na, unsigned nd, const BP2DAngle *ang, int plant, long *staged) {
     outside = 0;
+    others_fit = plant != 3;
     lds_base = 1u << 28;
     for (int Y0 = 0; Y0 < (int)h; Y0 += 64 / LX * TY)
         for (int X0 = 0; X0 < (int)w; X0 += LX * TX)
             for (unsigned a = 0; a < na; ++a) {
                 const BP2DAngle c = ang[a];
                 for (int lane = 0; lane < 64; ++lane) {
-                    """ + host(corners).replace("const float cy1 =", "float cy1 =").replace(
-                        "const bool whole =", "bool whole =") + r"""
-                    if (plant == 1) cy1 = cy0;
-                    """ + ("if (plant == 2) whole = true;" if "bool whole" in corners else "") + r"""
+                    """ + host(corners) + r"""
                     const int f = """ + call + r""";
                     if (!(f >> 20)) break;
                     if (lane == 0) ++*staged;
@@ -306,14 +312,16 @@ RAGGED = {"par": ("par", 130, 70, 200, 45, 0, 0), "fan": ("fan", 129, 97, 190, 6
 def test_bp2d_taps_inside_staged_footprint(lib, case, form):
     kind, w, h, nd, na, sod, odd = RAGGED[case]
     assert check2d(lib, kind, form, w, h, nd, na, sod, odd) == 0
+    # an angle beside it whose whole tile's interval is too long
+    assert check2d(lib, kind, form, w, h, nd, na, sod, odd, plant=3) == 0
 
 
 def test_bp2d_planted_first_row_footprint_is_caught(lib):
     assert check2d(lib, "fan", "32x32", 128, 96, 190, 60, 500.0, 300.0, plant=1) > 0
 
 
-def test_bp2d_planted_unclamped_cut_tile_is_caught(lib):
-    """Lanes past the slice of a tile that its edge cuts, without the clamp."""
+def test_bp2d_planted_cut_corners_are_caught(lib):
+    """Lanes past the edge of a slice against the footprint of those inside."""
     assert check2d(lib, "par", "32x32", 130, 70, 200, 45, 0, 0, plant=2) > 0
 
 
