@@ -114,13 +114,15 @@ def test_few_rows_take_the_gather(rules, shape, level):
 
 @pytest.mark.parametrize("shape, rays", [
     ((64, 64, 64, 90, 96, 96), 2), ((64, 64, 1, 30, 96, 1), 1), ((64, 64, 48, 90, 83, 64), 1),
-    ((128, 128, 48, 90, 166, 64), 1), ((256, 256, 96, 24, 332, 128), 2), ((512, 512, 512, 720, 768, 768), 4)])
+    ((128, 128, 48, 90, 166, 64), 1), ((256, 256, 96, 24, 332, 128), 2), ((512, 512, 512, 720, 768, 768), 4),
+    # the shapes whose values are checked with 1, 3 and 4 rays per lane
+    ((12, 12, 70, 300, 56, 64), 1), ((14, 12, 150, 300, 66, 192), 3), ((12, 13, 200, 300, 60, 251), 4)])
 def test_columns_where_they_are_faster(rules, shape, rays):
     assert cols_rays(rules, shape) == rays
 
 
 @pytest.mark.parametrize("shape, rays", [
-    ((400, 391, 130, 300, 513, 140), 3), ((512, 512, 48, 90, 665, 64), 1), ((256, 256, 48, 360, 332, 64), 0),
+    ((400, 391, 130, 300, 513, 140), 3), ((12, 14, 190, 300, 64, 190), 3), ((512, 512, 48, 90, 665, 64), 1), ((256, 256, 48, 360, 332, 64), 0),
     ((512, 512, 48, 360, 665, 64), 0)])
 def test_level_rays(rules, shape, rays):
     """64 rows of a full chip: one ray per lane up to 32768 waves."""

@@ -2,9 +2,8 @@
 (ASTRA_AMD_BP3D_LDS=1) against the kernel that reads the taps from global
 memory: same taps, weights and order of sums, so the volumes are equal bit
 for bit.  Cases cover the three kernel kinds (cone fr^2 and FDK weighting,
-cone 2d_weighting, par3d), LDS row layouts (odd or padded row lengths),
-SET / ADD and the SIRT update, more than 256
-angles per launch (two footprint groups), volumes whose edge blocks are
+cone 2d_weighting, par3d), SET / ADD and the SIRT update, more than 256
+angles per launch (three footprint groups), volumes whose edge blocks are
 partly outside, and a source close enough that footprints overflow the
 tile (those angles fall back to global memory).
 """
@@ -29,18 +28,16 @@ def _case(kind, nx, ny, nz, na, nu, nv, sod=300.0, odd=200.0):
 
 CASES = [
     ("cone", 40, 36, 28, 30, 64, 48, 300.0, 200.0),
-    ("cone", 33, 47, 19, 300, 72, 40, 300.0, 200.0),    # two footprint groups, ragged blocks
+    ("cone", 33, 47, 19, 300, 72, 40, 300.0, 200.0),    # three footprint groups, ragged blocks
     ("par3d", 45, 38, 21, 50, 64, 32, 0, 0),
     ("cone", 48, 48, 32, 24, 96, 96, 40.0, 400.0),      # near source: tiles overflow
 ]
 
 
-@pytest.mark.parametrize("pitch", ["-1", "0", "8", "3"], ids=["odd_rows", "pm0", "pm8", "pm3"])
 @pytest.mark.parametrize("case", CASES, ids=["cone", "cone_groups", "par3d", "cone_overflow"])
-def test_lds_bp_equals_global_bp(case, pitch, monkeypatch):
+def test_lds_bp_equals_global_bp(case, monkeypatch):
     kind, nx, ny, nz, na, nu, nv, sod, odd = case
     astra, vg, pg, proj = _case(kind, nx, ny, nz, na, nu, nv, sod, odd)
-    monkeypatch.setenv("ASTRA_AMD_BP3D_LDS_PITCH", pitch)
     out = {}
     for lds in (False, True):
         monkeypatch.setenv("ASTRA_AMD_BP3D_LDS", "1" if lds else "0")

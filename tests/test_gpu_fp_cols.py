@@ -23,9 +23,9 @@ CASES = {
     "too_wide_rows": ("cone", (24, 24, 60), 12, 40, 90, 1.0, 4.5, 120.0, 10.0),
     "par3d_129_rows": ("par3d", (33, 30, 90), 14, 45, 129, 1.1, 0.9, 0, 0),
     "rays_1": ("cone", (12, 12, 70), 300, 56, 64, 1.0, 1.5, 60.0, 5.0),
-    "rays_3": ("cone", (14, 12, 150), 90, 66, 192, 1.0, 1.0, 200.0, 60.0),
-    "rays_3_par": ("par3d", (12, 14, 190), 88, 64, 190, 1.0, 1.0, 0, 0),
-    "rays_4": ("cone", (12, 13, 200), 80, 60, 251, 1.0, 1.0, 260.0, 80.0),
+    "rays_3": ("cone", (14, 12, 150), 300, 66, 192, 1.0, 1.0, 200.0, 60.0),
+    "rays_3_par": ("par3d", (12, 14, 190), 300, 64, 190, 1.0, 1.0, 0, 0),
+    "rays_4": ("cone", (12, 13, 200), 300, 60, 251, 1.0, 1.0, 260.0, 80.0),
 }
 
 
