@@ -665,8 +665,8 @@ void launch_fp(const Batch2D &b, int cfg, const float *sinos, float *out, int mo
 
 // FP candidates: kFPDB tilings (0..2), the LDS-staged one (3) and the
 // kFPDB tilings with two detectors per thread (4..6).  The autotuner times
-// the first four (48 slices of 128 to 1024, per iteration: gathers 3.8 ms,
-// staged 1.4 ms with 4 angles per wave, 1.45 with 3, 1.6 with 2); the
+// the first four (48 slices of 128 to 1024, per iteration: gathers 3.7 ms,
+// staged 1.54 ms with 4 angles per wave, 1.61 with 3, 1.83 with 2); the
 // pairs never won (197 vs 200 slices/s on 4096 slices) and run by request
 // only.
 constexpr int kFPCandidates = 7;
@@ -676,8 +676,8 @@ constexpr int kFPTimed = 4;
 // every tap from global memory, 3..5 from LDS-staged footprints, 6..8 from
 // global memory two rows per load.  The autotuner times 0..5 (the row
 // pairs never won: 175 vs 173 slices/s at best).  48 slices of 128 to 1024,
-// per iteration: gathers 2.35 ms, staged 1.45 ms with 8 rows, 1.8 with 4;
-// tiles of 32 x 16 pixels per wave 1.42, not worth a form of their own.
+// per iteration: gathers 2.37 ms, staged 1.45 ms with 8 rows, 1.83 with 4;
+// tiles of 32 x 16 pixels per wave 2 % less, not worth a form of their own.
 constexpr int kBPCandidates = 9;
 constexpr int kBPTimed = 6;
 

@@ -301,8 +301,10 @@ __device__ __forceinline__ void bp2d_column(int X, int Y0, unsigned w, unsigned 
 // and after its own range add exact zeros), so the values equal
 // fp2d_value's.
 // Bound by issue (VALU 10 per sample) and by the second round of waves that
-// does not fill the GPU, no unit saturated.  FP of 1024^2 / 720 x 1536, fan:
-// 719 us with gathers, 276 to 300 here (16 slices per chunk 276, 8: 300).
+// does not fill the GPU, no unit saturated; the 128 registers of 4 waves per
+// SIMD do not hold the chunk in flight of 2 or 3 angles (spilled: parallel 23
+// and 47, fan 8 and 14 registers).  FP of 1024^2 / 720 x 1536, fan: 719 us
+// with gathers, 280 to 300 here; of 777 x 641 / 501 x 1013, parallel, 128.
 constexpr int kFp2SC = 16;      // slices per staged chunk
 constexpr int kFp2Row = 128;    // texels per staged slice row; or half the
                                 // slices and twice the texels
@@ -561,9 +563,9 @@ __device__ __forceinline__ void fp2d_wave(int d0, int a0, unsigned na, unsigned 
 // Lanes in 8 x 8 squares: the footprint is short for the updates it serves,
 // and the taps of neighbouring lanes share LDS words.
 // Bound by the VALU (parallel 7, fan 11 instructions per update, the fan's
-// reciprocal at a quarter of the rate): BP of 1024^2 / 720 x 1536 338 -> 225
+// reciprocal at a quarter of the rate): BP of 1024^2 / 720 x 1536 359 -> 240
 // us (fan, 10.7 clocks per update and CU), of 777 x 641 / 501 x 1013 209 ->
-// 79 us (parallel, 5.6).
+// 82 us (parallel, 5.6).
 // With LX = 64 and TX = 1 the taps, weights and the order of the sums are
 // those of bp2d_column, so both give the same floats.
 constexpr int kBp2KA = 4;     // angles per staged block

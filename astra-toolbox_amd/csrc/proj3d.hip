@@ -1237,9 +1237,11 @@ int bp_zs() {
 // planes, 16 z voxels per thread), chunks of 90 / 180 / 240 / 360 / 720:
 // 49.5 / 48.6 / 48.2 / 48.7 / 49.3 ms with gathers of row pairs, chunks of
 // 180 / 240 / 360 / 720: 40.1 / 39.6 / 39.5 / 39.5 ms with staged tiles of the
-// plain planes (1.7 GB).  So: 40 angles from 8 GiB
-// of padded projections on; below that, equal chunks of at most 1.2 GB of
-// planes (a single launch below 1.2 GB); in every output mode.
+// plain planes (1.7 GB).  So: 40 angles from 8 GiB of padded projections on;
+// below that, equal chunks of at most 1.2 GB of planes (a single launch below
+// 1.2 GB); in every output mode.  The lines are the gather's: staged tiles at
+// 1024^3 take 950 / 949 / 949 / 945 / 944 / 874 ms with 40 / 80 / 120 / 240 /
+// 480 / 1440 angles.
 // ASTRA_AMD_BP3D_ACHUNK=<angles> forces a chunk size (0: default rule; read
 // at every call, so a process can change it between calls).
 unsigned bp_achunk(size_t pair_bytes, unsigned na) {
