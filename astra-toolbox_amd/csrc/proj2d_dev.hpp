@@ -389,6 +389,9 @@ __device__ __forceinline__ void fp2d_wave(int d0, int a0, unsigned na, unsigned 
             if (FAN && m[j]) {
                 const double den = G.r[V] - G.p0[V] - (fdet - 0.5) * G.u[V];
                 const unsigned long long neg = __ballot(mine[j] && den < 0.0);
+                // farther positions (rays nearly along the slices; NaN where den
+                // is 0) round by more than the intervals' margin
+                simple = simple && !__ballot(mine[j] && !(fmaf(fabsf(R[j].a), (float)nsl, fabsf(R[j].c)) < 8e4f));
                 const int first = __builtin_ctzll(m[j]), last = 63 - __builtin_clzll(m[j]);
                 simple = simple && (neg == 0 || neg == m[j]) && __builtin_popcountll(m[j]) == last - first + 1;
                 // the other lanes follow the nearest one
@@ -434,7 +437,7 @@ __device__ __forceinline__ void fp2d_wave(int d0, int a0, unsigned na, unsigned 
                 tmin = fminf(tmin, fminf(tf, tl));
                 tmax = fmaxf(tmax, fmaxf(tf, tl));
             }
-            // 0.01: far beyond the rounding of the rays in between
+            // 0.01: beyond the rounding of the rays in between (of a and c, 2 x 2^-24 of 8e4)
             pclip = (tmin < 0.51f || tmax > hi_t - 0.01f) ? 1 : 0;
             plo = cvt_floor(clamp_pad(tmin - 0.01f, hi_t));
             phi = cvt_floor(clamp_pad(tmax + 0.01f, hi_t)) + 1;

@@ -2,7 +2,9 @@
 samples in the same order, so the same floats.  Slices and detectors around a
 wave's 64 detectors and a chunk's 16 slices, one, two and three angles per
 wave (by the number of waves), rays along both axes in one wave, detectors
-wide enough that a chunk exceeds its buffer, sub-rays, infinities."""
+wide enough that a chunk exceeds its buffer, sub-rays, infinities, and a
+source next to or on the detector's line, whose rays run along the slices
+(positions that round by texels, or are NaN)."""
 import numpy as np
 import pytest
 
@@ -19,6 +21,8 @@ pytestmark = pytest.mark.gpu
     ("fan", 97, 64, 400, 720, 0.3, 1),
     ("fan", 24, 33, 1501, 705, 0.1, 1),
     ("wide", 130, 129, 30, 300, 2.0, 3),
+    ("steep", 200, 210, 6, 64, 0.9, 1),
+    ("steep", 97, 300, 6, 200, 0.1, 2),
 ])
 def test_staged_equals_gather(monkeypatch, geom, w, h, na, nd, du, ss):
     import torch
@@ -28,6 +32,9 @@ def test_staged_equals_gather(monkeypatch, geom, w, h, na, nd, du, ss):
     vg = astra.create_vol_geom(h, w)
     if geom == "par":
         pg = astra.create_proj_geom("parallel", du, nd, ang)
+    elif geom == "steep":
+        gaps = [1e-1, 1e-3, 1e-4, 1e-5, 0.0, 3.0]
+        pg = astra.create_proj_geom("fanflat_vec", nd, np.array([[3.3, 7.5, 3.0, 7.5 - g, du, 0.0] for g in gaps]))
     else:
         sod = max(w, h) * (0.8 if geom == "wide" else 2.0)
         pg = astra.create_proj_geom("fanflat", du, nd, ang, sod, 0.1 * sod)

@@ -332,3 +332,61 @@ def test_bp2d_taps_inside_staged_footprint_batched_sizes(lib, case):
     origin-detector N), 8 rows per thread."""
     kind, w, h, nd, na, sod, odd = case
     assert check2d(lib, kind, "rows8", w, h, nd, na, sod, odd) == 0
+
+
+def fan_wave(src, det0, u, n, w, h):
+    """Float32 (a, c) of `ray2d` for n rays along the rows (V): position
+    a s + c at slice s, from a source and detector pixels det0 + k u."""
+    k = np.arange(n)
+    p0, p1 = det0[0] + k * u[0], det0[1] + k * u[1]
+    with np.errstate(all="ignore"):
+        a = -(src[0] - p0) / (src[1] - p1)
+        c = a * (-0.5 * h + 0.5) + p0 + p1 * a + 0.5 * w - 0.5 + 2
+    return a.astype(f32), c.astype(f32), src[1] - p1
+
+
+def fp2d_rule():
+    """The staged 2D FP's margin and its limit of |a| n + |c|."""
+    src = source("proj2d_dev.hpp")
+    margin = re.search(r"plo = cvt_floor\(clamp_pad\(tmin - ([\d.]+)f", src).group(1)
+    limit = re.search(r"!\(fmaf\(fabsf\(R\[j\]\.a\), \(float\)nsl, fabsf\(R\[j\]\.c\)\) < (\w+)f\)", src)
+    return float(margin), float(limit.group(1)) if limit else np.inf
+
+
+def outside_interval(a, c, den, h, hi, margin, limit):
+    """Samples of a staged wave whose texel is not between those of its first
+    and last ray; 0 where the wave is not staged."""
+    if not ((den > 0).all() or (den < 0).all() or (den >= 0).all()):
+        return 0
+    with np.errstate(all="ignore"):
+        if limit < np.inf and not (np.abs(a) * f32(h) + np.abs(c) < limit).all():
+            return 0
+        s = np.arange(h, dtype=f32)[:, None]
+        t = (a.astype(np.float64) * s + c).astype(f32)  # one fused multiply-add
+    ends = t[:, [0, -1]]
+    lo = np.fmin.reduce(ends, axis=1, keepdims=True, initial=f32(np.inf))
+    hi_ = np.fmax.reduce(ends, axis=1, keepdims=True, initial=f32(-np.inf))
+    clamp = lambda x: np.fmin(np.fmax(x, f32(0.5)), f32(hi))
+    plo, phi = np.floor(clamp(lo - f32(margin))), np.floor(clamp(hi_ + f32(margin)))
+    q = np.floor(np.where(np.isnan(t), 0, clamp(t)))  # NaN converts to texel 0
+    return int(np.count_nonzero((q < plo) | (q > phi)))
+
+
+@pytest.mark.parametrize("gap", [100.0, 3.0, 1e-1, 1e-3, 1e-4, 1e-5, 0.0])
+def test_fp2d_positions_inside_staged_interval(gap):
+    """Rays of a fan whose source is `gap` pixels from its detector's line,
+    down to on it: the steeper they are, the more their positions round."""
+    margin, limit = fp2d_rule()
+    bad = 0
+    for w, h, v in ((512, 512, 7.5), (1024, 900, -300.5), (97, 2000, 0.25)):
+        for du in (1.0, 0.1, 0.013):
+            a, c, den = fan_wave((3.3, v), (3.3 - 20 * du, v - gap), (du, 0.0), 64, w, h)
+            bad += outside_interval(a, c, den, h, w + 2.5, margin, limit)
+            a, c, den = fan_wave((3.3, v), (3.3 - 20 * du, v - gap), (du, -gap / 80), 64, w, h)
+            bad += outside_interval(a, c, den, h, w + 2.5, margin, limit)
+    assert bad == 0
+
+
+def test_fp2d_planted_steep_rays_are_caught():
+    a, c, den = fan_wave((3.3, 7.5), (-16.7, 7.5 - 1e-5), (1.0, 0.0), 64, 512, 512)
+    assert outside_interval(a, c, den, 512, 514.5, fp2d_rule()[0], np.inf) > 0
