@@ -291,9 +291,10 @@ void fp3d_cols_copy(const Geom3D &g, const float *vol, float *cols, hipStream_t 
 namespace {
 // Rows one chunk of group `grp` can need with r rays per lane: the rays'
 // spread, their drift over the chunk, and the two taps with the margins of
-// params().
+// params().  Steeper rays' heights, up to 4000 slices times their slope, round
+// by more than those margins in fp32.
 bool fits(const ColsBound &b, int r) {
-    return (64 * r - 1) * b.spread + (kSl - 1) * b.slope + 3.1 <= 64.0 * (r + 1);
+    return b.slope <= 10.0 && (64 * r - 1) * b.spread + (kSl - 1) * b.slope + 3.1 <= 64.0 * (r + 1);
 }
 double waves(const Geom3D &g, int grp, int r) {
     return (double)g.nu * g.dir_count[grp] * ((g.nv + 64 * r - 1) / (64 * r));

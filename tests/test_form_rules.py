@@ -129,6 +129,14 @@ def test_level_rays(rules, shape, rays):
     assert cols_rays(rules, shape, level=True) == rays
 
 
+@pytest.mark.parametrize("slope, rays", [(8.0, 2), (10.0, 2), (10.1, 0), (15.0, 0)])
+def test_steep_rays_take_the_gather(rules, slope, rays):
+    """A chunk's window of rows holds the outermost rays' heights with 0.01
+    rows to spare; |a| n + |c| of 8 x 10^4 rounds by half of that in fp32."""
+    n = (ctypes.c_uint * 6)(64, 64, 64, 90, 96, 96)
+    assert rules.cols_rays(n, *(ctypes.c_double(x) for x in (0.5, 0.4, slope))) == rays
+
+
 # n^3 volume, angles, columns = rows, pixel, source and detector distance;
 # share of blocks and angles whose footprint exceeds the staged tile, counted
 # over all of them (every eleventh angle)
