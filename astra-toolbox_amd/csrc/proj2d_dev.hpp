@@ -303,7 +303,7 @@ __device__ __forceinline__ void bp2d_column(int X, int Y0, unsigned w, unsigned 
 // Bound by issue (VALU 10 per sample) and by the second round of waves that
 // does not fill the GPU, no unit saturated; the 128 registers of 4 waves per
 // SIMD do not hold the chunk in flight of 2 or 3 angles (spilled: parallel 23
-// and 47, fan 8 and 14 registers).  FP of 1024^2 / 720 x 1536, fan: 719 us
+// and 47, fan 8 and 15 registers).  FP of 1024^2 / 720 x 1536, fan: 719 us
 // with gathers, 280 to 300 here; of 777 x 641 / 501 x 1013, parallel, 128.
 constexpr int kFp2SC = 16;      // slices per staged chunk
 constexpr int kFp2Row = 128;    // texels per staged slice row; or half the
